@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes as C
 from dataclasses import dataclass
+from functools import lru_cache
 from typing import Optional
 
 import torch
@@ -25,9 +26,16 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+# The host side of a call must cost less than a small kernel (9 us): through torch's Python objects
+# (current_stream(), device objects) one gemm call took 14.7 us.  The raw stream and the tensors'
+# flags say the same.
+_get_device = torch._C._cuda_getDevice
+_get_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 def _stream(stream) -> int:
     if stream is None:
-        return torch.cuda.current_stream().cuda_stream
+        return _get_raw_stream(_get_device())
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
@@ -36,7 +44,7 @@ def _stream(stream) -> int:
 def _need(t: torch.Tensor, name: str, dtypes: tuple) -> None:
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{name} must be a device tensor (got {t.device})")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
@@ -54,7 +62,10 @@ def workspace(nbytes: int, device: Optional[torch.device] = None, stream=None) -
     ready flags never meet.  Growing synchronizes the device twice: before the old buffer is
     released (kernels still queued on any stream may use it) and after the zero fill (issued on
     torch's current stream, the kernels run on `stream`).  Grow outside graph capture."""
-    dev = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
+    if isinstance(device, torch.device):
+        dev = device
+    else:
+        dev = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
     key = (idx, _stream(stream))
     ws = _workspaces.get(key)
@@ -97,6 +108,11 @@ class GroupWords:
         return GroupWordsC(self.trellis.data_ptr(), self.suh.data_ptr(), self.svh.data_ptr(), m)
 
 
+@lru_cache(maxsize=4096)
+def _gemm_workspace_bytes(M: int, N: int, K: int) -> int:
+    return lib.hx_exl3_gemm_workspace_size(M, N, K)
+
+
 def gemm(y: torch.Tensor, x: torch.Tensor, w: GroupWords, M: int, N: int, K: int, bits: int, y_fp32: bool = False,
          stream=None, a_had: Optional[torch.Tensor] = None, mcg: bool = False) -> int:
     """y = svh . H_N(H_K(x . suh) . W_hat).  Returns 90 when the small-M GEMV ran, 1 for MFMA."""
@@ -110,11 +126,11 @@ def gemm(y: torch.Tensor, x: torch.Tensor, w: GroupWords, M: int, N: int, K: int
         raise ValueError("GroupWords shapes do not match K, N, bits")
     if a_had is not None:
         _need(a_had, "a_had", (torch.float16,))
-    nbytes = lib.hx_exl3_gemm_workspace_size(M, N, K)
-    ws = workspace(nbytes, x.device, stream) if (M <= GEMV_MAX_M or a_had is None) else None
+    st = _stream(stream)
+    ws = workspace(_gemm_workspace_bytes(M, N, K), x.device, st) if (M <= GEMV_MAX_M or a_had is None) else None
     gw = w.c()
-    return check(lib.hx_exl3_gemm(y.data_ptr(), x.data_ptr(), C.byref(gw), M, N, K, bits, int(y_fp32),
-                                  _stream(stream), _ptr(a_had), int(mcg), _ptr(ws), ws.numel() if ws is not None else 0),
+    return check(lib.hx_exl3_gemm(y.data_ptr(), x.data_ptr(), C.byref(gw), M, N, K, bits, int(y_fp32), st,
+                                  _ptr(a_had), int(mcg), _ptr(ws), ws.numel() if ws is not None else 0),
                  "hx_exl3_gemm")
 
 
