@@ -294,6 +294,15 @@ HX_INLINE void quarter_affine(const uint32_t* r, uint32_t* out)
     quarter_affine_pairs<BITS>(r, M, out);
 }
 
+// Keeps the 16 decoded registers computed here: without it the compiler sinks a step's decode behind
+// the branch of the step's input read, past the refill of the ring slot it reads from.
+HX_INLINE void pin_regs16(uint32_t* d)
+{
+    asm volatile("" : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]), "+v"(d[4]), "+v"(d[5]), "+v"(d[6]), "+v"(d[7]),
+                      "+v"(d[8]), "+v"(d[9]), "+v"(d[10]), "+v"(d[11]), "+v"(d[12]), "+v"(d[13]), "+v"(d[14]),
+                      "+v"(d[15]));
+}
+
 // MFMA B operand (nh, kh) of a decoded quarter: column 8nh+q, k = 8kh + 0..7, i.e. local positions
 // 2kh + 4nh + 8j + {0, 1} for j = 0..3: pairs I0 + 4j, I0 = kh + 2nh, stored at out[4 I0 + j] (qpos),
 // so an operand is four consecutive registers and needs no moves.
@@ -310,140 +319,96 @@ HX_INLINE hx_h8 quarter_operand(const uint32_t* d)
     return __builtin_bit_cast(hx_h8, v);
 }
 
-// Input transform of rows [0, M) over k in [k0, k0 + kc) into LDS as fp16:
-//   a = fp16(H128(fp16(x . suh)))   (reference had_hf_r_128_inner<true,false>)
-// When pre_transformed, x already holds a (copied as is, read with device-coherent loads because
-// another workgroup of the same launch may have produced it).
+// ---- input transform of rows [0, M) over k in [k0, k0 + kc) into LDS as fp16
 //
-// Job j (row m, 128-wide block b) is done by wave j % 4.  The loads of a wave's first IN_PRE jobs are
-// issued separately (input_issue) so that a caller can put them ahead of the tile prefetch: the
-// vector-memory counter completes in issue order, so an input load issued after the prefetch would
-// make the transform wait for every prefetched tile.
-constexpr int IN_PRE = 4;
+//   a = fp16(H128(fp16(x . suh)))   (reference had_hf_r_128_inner<true,false>)
+//
+// on the matrix cores, 16 (row, 128-wide block) pairs per group: the group's pairs are the 16 columns
+// of the product, so one token's 16 blocks fill it as well as 16 tokens' rows of one block.  H128
+// splits over the 4 32-wide parts kk of a block: for output n = 16 nb + r the sign of (n, k) is
+// popcount(n & k) & 1, and the bits of kk meet only bits 1 and 2 of nb.  So the part products P[nb & 1][kk]
+// (8 MFMAs, H's operand generated in registers: a fixed per-lane fragment times one sign per lane)
+// are added by two 4-point butterflies instead of 32 MFMAs with a sign per operand.  fp32 sums of exact
+// products, one fp16 rounding after the 1/sqrt(128) scale.  A wave-wide butterfly per pair (64 lanes,
+// 12 shuffles) took 5 times the instructions: the transform, repeated by every column group,
+// was 10-30 % of the VALU work of the decode kernels (lm_head at M = 1: 4.2 VALU instructions per weight
+// against 3.3 in its loop).
+// Lane l = 16g + c loads k = 32 kk + 8g + 0..7 of pair c and ends with columns 16 nb + 4g + 0..3 of it.
+//
+// input_load is separate so that a caller can issue the loads of a wave's first group ahead of the tile
+// prefetch: the vector-memory counter completes in issue order, so an input load issued after the
+// prefetch would make the transform wait for every prefetched tile.
+typedef _Float16 hx_h8u __attribute__((ext_vector_type(8), aligned(4)));  // rows of any 4-byte alignment
 
 struct InputRegs {
-    uint32_t xv[IN_PRE];
-    uint32_t sv[IN_PRE];
+    hx_h8 x[4], s[4];
 };
 
-HX_INLINE uint32_t input_word(const _Float16* x, const int* rows, int M, int K, int k0, int blocks, int job, int lane,
-                              bool pre_transformed)
+HX_INLINE void input_load(InputRegs& r, const _Float16* x, const int* rows, const _Float16* suh, int jobs, int blocks,
+                          int K, int k0, int job0)
 {
-    const int m = job / blocks, b = job % blocks;
-    const int k = k0 + b * 128 + 2 * lane;
+    const int lane = threadIdx.x & 63, g = lane >> 4;
+    const int job = min(job0 + (lane & 15), jobs - 1);  // pairs past the last repeat it (not stored)
+    const int m = job / blocks, k = k0 + (job - m * blocks) * 128 + 8 * g;
     const size_t row = rows ? (size_t)rows[m] : (size_t)m;
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(x + row * K + k);
-    if (pre_transformed) return __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return *(hx_gu32*)src;
-}
-
-HX_INLINE void input_issue(InputRegs& r, const _Float16* x, const int* rows, const _Float16* suh, int M, int K, int k0,
-                           int kc, bool pre_transformed)
-{
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int blocks = kc >> 7;
 #pragma unroll
-    for (int i = 0; i < IN_PRE; ++i) {
-        const int job = wave + hx_nwaves() * i;
-        r.xv[i] = 0;
-        r.sv[i] = 0;
-        if (job < M * blocks) {
-            r.xv[i] = input_word(x, rows, M, K, k0, blocks, job, lane, pre_transformed);
-            if (!pre_transformed)
-                r.sv[i] = *(hx_gu32*)(suh + k0 + (job % blocks) * 128 + 2 * lane);
-        }
+    for (int kk = 0; kk < 4; ++kk) {
+        r.x[kk] = *reinterpret_cast<const hx_h8u*>(x + row * K + k + 32 * kk);
+        r.s[kk] = *reinterpret_cast<const hx_h8u*>(suh + k + 32 * kk);
     }
 }
 
-HX_INLINE uint32_t input_transform(uint32_t xv, uint32_t sv, bool pre_transformed)
+HX_INLINE void input_store(uint32_t* a_lds, const InputRegs& r, int jobs, int job0)
 {
-    if (pre_transformed) return xv;
-    hx_h2 p = u32_as_h2(xv) * u32_as_h2(sv);
-    float v0 = (float)p.x, v1 = (float)p.y;
-    hx_had128_wave(v0, v1);
-    hx_h2 r = {(_Float16)v0, (_Float16)v1};
-    return h2_as_u32(r);
-}
-
-// The input transform of up to 16 rows at once on the matrix cores: per 128-k block, the rows'
-// fp16(x . suh) (rows >= M zero) times H128 as one 16 x 128 by 128 x 128 product, H generated in
-// registers (sign of (n, k) = popcount(n & k) & 1: a fixed per-lane fragment times one sign per
-// operand), fp32 accumulation of the exact +-products, one fp16 rounding after the 1/sqrt(128)
-// scale.  The same values as the butterfly (hx_had128_wave) up to the order of the fp32 additions;
-// for several rows it replaces a wave-wide butterfly per row and block with 32 MFMAs per block.
-// Lane l: A row l % 16, k = 32 kk + 8 (l / 16) + 0..7; C rows 4 (l / 16) + i, column 16 nb + l % 16.
-HX_INLINE void input_mfma(uint32_t* a_lds, const _Float16* x, const int* rows, const _Float16* suh, int M, int K,
-                          int k0, int kc, int ld = -1)
-{
-    if (ld < 0) ld = kc;  // row stride of the LDS rows (fp16)
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int c = lane & 15, g = lane >> 4;
-    const int blocks = kc >> 7;
-    uint32_t f[4];
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+    u4v f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const uint32_t s0 = __builtin_popcount(c & (2 * i) & 7) & 1, s1 = __builtin_popcount(c & (2 * i + 1) & 7) & 1;
         f[i] = (0x3c00u | (s0 << 15)) | ((0x3c00u | (s1 << 15)) << 16);
     }
-    const uint32_t base = (uint32_t)((c >> 3) & g & 1);
-    const bool live = c < M;
-    const _Float16* xr = x + (live ? (rows ? (size_t)rows[c] : (size_t)c) : 0) * K + 8 * g;
-    _Float16* al = reinterpret_cast<_Float16*>(a_lds);
-    for (int b = wave; b < blocks; b += hx_nwaves()) {
-        const int kb = k0 + b * 128;
-        hx_h8 av[4];
+    const uint32_t even = ((c >> 3) & g & 1) ? 0x80008000u : 0u, odd = (g >> 1) ? 0x80008000u : 0u;
+    const bool live = job0 + c < jobs;
+    _Float16* al = reinterpret_cast<_Float16*>(a_lds) + (size_t)(job0 + c) * 128 + 4 * g;
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            const hx_h8 sv = *reinterpret_cast<const hx_h8*>(suh + kb + 32 * kk + 8 * g);
-            hx_h8 xv = {};
-            if (live) xv = *reinterpret_cast<const hx_h8*>(xr + kb + 32 * kk);
-            av[kk] = xv * sv;
-        }
-        hx_f4 y[8];
-#pragma unroll
-        for (int nb = 0; nb < 8; ++nb) y[nb] = hx_f4{0.f, 0.f, 0.f, 0.f};
+    for (int nb0 = 0; nb0 < 2; ++nb0) {
+        const hx_h8 h = __builtin_bit_cast(hx_h8, f ^ (nb0 ? even ^ odd : even));
+        hx_f4 p[4];
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk)
+            p[kk] = __builtin_amdgcn_mfma_f32_16x16x32_f16(h, r.x[kk] * r.s[kk], hx_f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        const hx_f4 s0 = p[0] + p[1], d0 = p[0] - p[1], s1 = p[2] + p[3], d1 = p[2] - p[3];
+        const hx_f4 y[4] = {s0 + s1, d0 + d1, s0 - s1, d0 - d1};
 #pragma unroll
-            for (int nb = 0; nb < 8; ++nb) {
-                const uint32_t sgn = base ^ ((uint32_t)(nb & 1) & (uint32_t)(g >> 1)) ^ (uint32_t)((nb >> 1) & kk & 1) ^
-                                     (uint32_t)((nb >> 2) & (kk >> 1) & 1);
-                const uint32_t m = sgn ? 0x80008000u : 0u;
-                typedef uint32_t u4v __attribute__((ext_vector_type(4)));
-                const u4v bv = {f[0] ^ m, f[1] ^ m, f[2] ^ m, f[3] ^ m};
-                y[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[kk], __builtin_bit_cast(hx_h8, bv), y[nb], 0, 0, 0);
-            }
+        for (int q = 0; q < 4; ++q) {
+            hx_h4 v;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int m = 4 * g + i;
-            if (m < M) {
-#pragma unroll
-                for (int nb = 0; nb < 8; ++nb) al[m * ld + b * 128 + 16 * nb + c] = (_Float16)(y[nb][i] * HX_RSQRT128);
-            }
+            for (int i = 0; i < 4; ++i) v[i] = (_Float16)(y[q][i] * HX_RSQRT128);
+            if (live) *reinterpret_cast<hx_h4*>(al + 16 * (nb0 + 2 * q)) = v;
         }
     }
 }
 
-// Transform and store all jobs: the first IN_PRE per wave from r, the rest loaded here.
-HX_INLINE void input_finish(uint32_t* a_lds, const InputRegs& r, const _Float16* x, const int* rows,
-                            const _Float16* suh, int M, int K, int k0, int kc, bool pre_transformed)
+// Copy of an already transformed input (rows m of x, no gather), read with device-coherent loads because
+// another workgroup of the same launch produced it; job j (row, 128-wide block) is done by wave j % 4.
+HX_INLINE void input_copy(uint32_t* a_lds, const _Float16* x, int M, int K, int k0, int kc)
 {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int blocks = kc >> 7;
+    const int blocks = kc >> 7, jobs = M * blocks;
+    constexpr int B = 4;  // loads in flight per lane
+    for (int j0 = wave; j0 < jobs; j0 += B * hx_nwaves()) {
+        uint32_t v[B];
 #pragma unroll
-    for (int i = 0; i < IN_PRE; ++i) {
-        const int job = wave + hx_nwaves() * i;
-        if (job < M * blocks) {
-            const int m = job / blocks, b = job % blocks;
-            a_lds[(m * kc + b * 128) / 2 + lane] = input_transform(r.xv[i], r.sv[i], pre_transformed);
+        for (int i = 0; i < B; ++i) {
+            const int job = min(j0 + i * hx_nwaves(), jobs - 1), m = job / blocks;
+            v[i] = __hip_atomic_load(reinterpret_cast<const uint32_t*>(x + (size_t)m * K + k0 +
+                                                                       (job - m * blocks) * 128 + 2 * lane),
+                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-    }
-    for (int job = wave + hx_nwaves() * IN_PRE; job < M * blocks; job += hx_nwaves()) {
-        const int m = job / blocks, b = job % blocks;
-        const uint32_t xv = input_word(x, rows, M, K, k0, blocks, job, lane, pre_transformed);
-        const uint32_t sv =
-            pre_transformed ? 0u : *(hx_gu32*)(suh + k0 + b * 128 + 2 * lane);
-        a_lds[(m * kc + b * 128) / 2 + lane] = input_transform(xv, sv, pre_transformed);
+#pragma unroll
+        for (int i = 0; i < B; ++i)
+            if (j0 + i * hx_nwaves() < jobs) a_lds[(j0 + i * hx_nwaves()) * 64 + lane] = v[i];
     }
 }
 
@@ -546,26 +511,37 @@ __device__ __forceinline__ void gemv_range(const GemvArgs& g, int cg, int k0, in
     const int voff = lane_off + q * BITS * 4;
     const int row_bytes = tiles_n * NW * 4;
     auto soff = [&](int st) { return ((k0 + step_k(min(st, steps - 1))) >> 4) * row_bytes; };
+    // the wave's groups of 16 (row, block) pairs; the lead wave rotates with the workgroup (a short
+    // range has one group, and all co-resident workgroups would put it on the same SIMD)
+    const int jobs = g.M * nblk, vw = __builtin_amdgcn_readfirstlane((wave - (int)blockIdx.x) & (hx_nwaves() - 1));
     InputRegs in;
-    // several rows: the transform on the matrix cores (its loads are issued there)
-    constexpr bool MF_IN = MT >= 4;
-    if (!g.pre_transformed && !MF_IN) input_issue(in, g.x, g.rows, g.suh, g.M, g.K, k0, kc, false);
+    if (!g.pre_transformed && 16 * vw < jobs) input_load(in, g.x, g.rows, g.suh, jobs, nblk, g.K, k0, 16 * vw);
     if (steps > 0) {
 #pragma unroll
         for (int j = 0; j < PF; ++j) load_quarter_buf<BITS>(buf[j], rs, voff, soff(j));
     }
 
     before_input();
-    if (g.pre_transformed) input_issue(in, g.x, g.rows, g.suh, g.M, g.K, k0, kc, true);
-    if (MF_IN && !g.pre_transformed) input_mfma(a_lds, g.x, g.rows, g.suh, g.M, g.K, k0, kc);
-    else input_finish(a_lds, in, g.x, g.rows, g.suh, g.M, g.K, k0, kc, g.pre_transformed);
+    if (g.pre_transformed) {
+        input_copy(a_lds, g.x, g.M, g.K, k0, kc);
+    } else if (16 * vw < jobs) {
+        input_store(a_lds, in, jobs, 16 * vw);
+        for (int j0 = 16 * (vw + hx_nwaves()); j0 < jobs; j0 += 16 * hx_nwaves()) {
+            input_load(in, g.x, g.rows, g.suh, jobs, nblk, g.K, k0, j0);
+            input_store(a_lds, in, jobs, j0);
+        }
+    }
     hx_lds_barrier();
     after_input();
     if constexpr (AFFINE) {
         for (int m = wave; m < g.M && m < MT; m += hx_nwaves()) {
             const _Float16* row = reinterpret_cast<const _Float16*>(a_lds) + (size_t)m * kc;
             float v = 0.0f;
-            for (int k = lane; k < kc; k += 64) v += (float)row[k];
+            for (int k = 8 * lane; k < kc; k += 512) {
+                const hx_h8 h = *reinterpret_cast<const hx_h8*>(row + k);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v += (float)h[j];
+            }
 #pragma unroll
             for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
             if (lane == 0) asum[m] = v;
@@ -583,6 +559,10 @@ __device__ __forceinline__ void gemv_range(const GemvArgs& g, int cg, int k0, in
     const bool a_reads = ROW ? diag : (MT == 1 || (lane & 15) < g.M);
     const _Float16* arow = reinterpret_cast<const _Float16*>(a_lds) + (size_t)am * kc;
     hx_h8 a0 = {}, a1 = {};
+    // The step's input read goes ahead of its decode with several rows and a deep ring (the layer at 4
+    // tokens 117.4 -> 114.6 us); after it otherwise (one-token layer 41.9 us against 42.3 us with the
+    // read first, dense linear with 5 rows 14.46 us against 14.55 us).
+    constexpr bool A_FIRST = MT > 1 && PF > 2;
     // one group of PF steps; GUARD: the group runs past the range (only the last group can)
     auto group = [&](int st0, auto guard) {
         constexpr bool GUARD = decltype(guard)::value;
@@ -603,18 +583,23 @@ __device__ __forceinline__ void gemv_range(const GemvArgs& g, int cg, int k0, in
             // so every wait, is the same at every step
             const bool live = !GUARD || st < steps;
             uint32_t d[16];
-            if (live) {
-                quarter_wrap<BITS>(buf[j]);
-                if constexpr (AFFINE) quarter_affine<BITS>(buf[j], d);
-                else quarter_decode<BITS, CB>(buf[j], d);
-            }
-            load_quarter_buf<BITS>(buf[j], rs, voff, soff(st + PF));
-            if (live) {
+            auto read_a = [&] {
                 const int kl = step_k(st) + 16 * gq;
                 if (a_reads) {
                     a0 = *reinterpret_cast<const hx_h8*>(arow + kl);
                     a1 = *reinterpret_cast<const hx_h8*>(arow + kl + 8);
                 }
+            };
+            if (live) {
+                if constexpr (A_FIRST) read_a();
+                quarter_wrap<BITS>(buf[j]);
+                if constexpr (AFFINE) quarter_affine<BITS>(buf[j], d);
+                else quarter_decode<BITS, CB>(buf[j], d);
+                if constexpr (ROW || MT > 1) pin_regs16(d);
+            }
+            load_quarter_buf<BITS>(buf[j], rs, voff, soff(st + PF));
+            if (live) {
+                if constexpr (!A_FIRST) read_a();
                 acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, quarter_operand<0, 0>(d), acc0, 0, 0, 0);
                 acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, quarter_operand<0, 1>(d), acc0, 0, 0, 0);
                 acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, quarter_operand<1, 0>(d), acc1, 0, 0, 0);

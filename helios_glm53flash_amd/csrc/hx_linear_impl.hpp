@@ -39,7 +39,7 @@ __device__ void linear_epilogue(const float* colsum, hx_h2 sv, void* y, int M, i
 }
 
 template <int BITS, int CB, int MT>
-__global__ __launch_bounds__(GEMV_THREADS) void linear_gemv_kernel(GemvArgs g, const _Float16* svh, void* y,
+__global__ __launch_bounds__(GEMV_THREADS, 5) void linear_gemv_kernel(GemvArgs g, const _Float16* svh, void* y,
                                                                   bool y_fp32)
 {
     extern __shared__ uint32_t a_lds[];
@@ -65,7 +65,7 @@ HX_INLINE unsigned stream_owner(unsigned b, unsigned units, unsigned wgs) { retu
 // T = (N/128) * (K/128), group by group.  A group met by several workgroups is finished by the last
 // to arrive, which adds the partials in workgroup order (deterministic); the others publish theirs.
 template <int BITS, int CB>
-__global__ __launch_bounds__(GEMV_THREADS) void linear_gemv_stream_kernel(GemvArgs g, const _Float16* svh, void* y,
+__global__ __launch_bounds__(GEMV_THREADS, 4) void linear_gemv_stream_kernel(GemvArgs g, const _Float16* svh, void* y,
                                                                          bool y_fp32)
 {
     extern __shared__ uint32_t a_lds[];

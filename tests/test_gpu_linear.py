@@ -73,6 +73,29 @@ def test_gemv_parity(hx, M, bits, cb):
     assert_close(got, ref, what=f"gemv M={M} bits={bits} cb={cb}")
 
 
+@pytest.mark.parametrize("M,K", [(1, 128), (1, 2048), (1, 2176), (2, 1152), (3, 6400), (5, 384), (9, 1920), (16, 128)])
+def test_gemv_input_transform_groups(hx, M, K):
+    """The input transform's groups of 16 (row, block) pairs: one pair, exactly one group, remainders, more
+    groups than waves; split ranges that are not a multiple of a group."""
+    _, got, ref = _run_linear(hx, M, K, 256, 3, 2, True, seed=M + K)
+    assert_close(got, ref, what=f"gemv M={M} K={K}")
+
+
+def test_gemv_input_at_4_byte_alignment(hx):
+    import torch
+    from oracle import oracle as O
+    K, N, bits = 1024, 256, 4
+    tr, suh, svh = make_linear(8, K, N, bits)
+    x = make_x(9, 3, K)
+    at2 = [torch.cat([torch.zeros(2, dtype=torch.float16), torch.from_numpy(v).reshape(-1)]).cuda()[2:]
+           for v in (x, suh)]  # contiguous, 4 bytes past a 16-byte boundary
+    w = hx.GroupWords(_dev(tr, torch.int16), at2[1], _dev(svh), hx.MUL1)
+    y = torch.empty((3, N), dtype=torch.float32, device="cuda")
+    hx.gemm(y, at2[0], w, 3, N, K, bits, True)
+    torch.cuda.synchronize()
+    assert_close(y.cpu().numpy(), O.linear(x, tr, suh, svh, K, N, bits, 2, out_f16=False), what="4-byte alignment")
+
+
 def test_gemv_fp16_out_and_repeat(hx):
     # second call reuses the workspace counters (must have been reset by the first)
     for _ in range(3):
