@@ -6,10 +6,9 @@
 //   M <= 8   gemv: one workgroup per output column n; its 4 waves split K, each lane takes 8
 //            consecutive k per step (16-byte loads of w and x), v_dot2_f32_f16 accumulation, the
 //            wave sums added in wave order.
-//   M > 8    direct-load MFMA: each wave computes a 32 x 32 block with v_mfma_f32_16x16x32_f16; both
-//            operands are contiguous along k, so a lane's MFMA fragment (8 halves) is one 16-byte
-//            load from L2, no LDS staging.
-#include "hx_device.hpp"
+//   M > 8    MFMA, the waves of a workgroup split K (gemm_nt_split_kernel): each streams both operands of
+//            its k range through LDS by itself, and the waves' sums are added at the end.
+#include "hx_mfma.hpp"
 #include "hx_kernels.hpp"
 
 namespace hx {
@@ -72,50 +71,147 @@ __global__ __launch_bounds__(256) void gemv_nt_kernel(const _Float16* x, const _
     }
 }
 
-// Workgroup = 4 waves stacked along m: rows 128*bx + 32*wave .. +31, columns 32*by .. +31.
-__global__ __launch_bounds__(256) void gemm_nt_mfma_kernel(const _Float16* x, const _Float16* w, void* y, int M,
-                                                           int N, int K, bool y_fp32, bool add)
+// One workgroup: rows 16 RB * bx + .., columns 16 CB * by + ..; its KS waves take equal k ranges of the
+// same tile, and their fp32 sums are added pairwise through LDS (wave w + wave w + h, h = KS/2, .., 1: a
+// fixed order).  N is small here (a router's 64-288 experts), so tiles alone leave the chip idle, and one
+// wave per 32 x 32 block over all of K waited a round trip of latency every few steps (115 us at
+// 4096 x 288 x 4096, 27 us at M = 16).  A wave has NB chunks of 64 k in LDS buffers of its own, filled
+// by buffer loads with an LDS destination (8 rows x 128 bytes each): no barrier, only its own loads to
+// wait for.  What bounds it is a CU's read path from L2: whole 128-byte lines come at 115 GB/s
+// per CU, the 64-byte halves that fragments loaded straight into MFMA layout touch at 37 GB/s (that
+// variant of this kernel: 45 us at M = 4096, 17 us at M = 33-512).
+// LDS rows are 64 halves with the 16-byte chunks of row r permuted by mf_swz(r) (hx_mfma.hpp).
+template <int RB, int CB, int KS, int NB>
+__device__ __forceinline__ void gemm_nt_split(const _Float16* x, const _Float16* w, void* y, int M, int N, int K,
+                                              bool y_fp32, bool add)
 {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int r0 = 128 * blockIdx.x + 32 * wave, c0 = 32 * blockIdx.y;
-    if (r0 >= M) return;  // whole wave past the last row (uniform)
-    const int lr = lane & 15, lk = 8 * (lane >> 4);
-    // fragment rows / columns of this lane (clamped: out-of-range rows and columns are not stored)
-    const _Float16* ap[2];
-    const _Float16* bp[2];
+    constexpr int ROWS = 16 * (RB + CB), NL = ROWS / 8;  // LDS rows and loads per chunk
+    static_assert(sizeof(hx_f4) * 64 * RB * CB * (KS / 2) <= sizeof(_Float16) * KS * NB * ROWS * 64, "sums fit the buffers");
+    extern __shared__ _Float16 buf[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int r0 = 16 * RB * blockIdx.x, c0 = 16 * CB * blockIdx.y;
+    const int nk = (K + 63) / 64, kq = (nk + KS - 1) / KS;  // chunks in all, per wave
+    const int q0 = wave * kq, n = min(nk, q0 + kq) - q0;
+    _Float16* wb = buf + (size_t)wave * NB * ROWS * 64;
+    const __amdgpu_buffer_rsrc_t rx = mf_rsrc(x + (size_t)r0 * K, (size_t)(M - r0) * K * sizeof(_Float16));
+    const __amdgpu_buffer_rsrc_t rw = mf_rsrc(w + (size_t)c0 * K, (size_t)(N - c0) * K * sizeof(_Float16));
+    // lane l of load i fetches, for LDS row r = 8i + l/8, the chunk that the permutation puts in slot l % 8;
+    // rows past the end (clamped) are computed but not stored; a chunk past K reads the next row's k or,
+    // past the end, zeros, and its MFMAs are skipped below
+    int voff[NL];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        ap[i] = x + (size_t)min(r0 + 16 * i + lr, M - 1) * K + lk;
-        bp[i] = w + (size_t)min(c0 + 16 * i + lr, N - 1) * K + lk;
+    for (int i = 0; i < NL; ++i) {
+        const int r = 8 * i + (lane >> 3), rr = i < 2 * RB ? min(r, M - r0 - 1) : min(r - 16 * RB, N - c0 - 1);
+        voff[i] = (int)(((size_t)rr * K + 8 * ((lane & 7) ^ mf_swz(r))) * sizeof(_Float16));
     }
-    hx_f4 acc[2][2];
+    auto load = [&](int p) {
+        const int q = q0 + p;
+        _Float16* d = wb + p % NB * ROWS * 64;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < NL; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(i < 2 * RB ? rx : rw,
+                                                     (__attribute__((address_space(3))) void*)(d + 512 * i), 16,
+                                                     voff[i], q * 128, 0, 0);
+    };
+    hx_f4 acc[RB][CB];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = hx_f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (int k = 0; k < K; k += 32) {
-        hx_h8 a[2], b[2];
+    for (int i = 0; i < RB; ++i)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            a[i] = *reinterpret_cast<const hx_h8*>(ap[i] + k);
-            b[i] = *reinterpret_cast<const hx_h8*>(bp[i] + k);
+        for (int j = 0; j < CB; ++j) acc[i][j] = hx_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int p = 0; p < NB; ++p)
+        if (p < n) load(p);
+    for (int p = 0; p < n; ++p) {
+        // chunk p has arrived once at most the loads of the later chunks in flight are outstanding
+        asm volatile("" ::: "memory");
+        if (n - p >= NB) __builtin_amdgcn_s_waitcnt(qt_vmcnt((NB - 1) * NL));
+        else __builtin_amdgcn_s_waitcnt(qt_vmcnt(0));
+        asm volatile("" ::: "memory");
+        const int q = q0 + p;
+        const _Float16* s = wb + p % NB * ROWS * 64;
+        hx_h8 f[2][RB + CB];
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (int i = 0; i < RB + CB; ++i)
+                f[kk][i] = *reinterpret_cast<const hx_h8*>(s + mf_off(16 * i + (lane & 15), 4 * kk + (lane >> 4)));
+        // every fragment is in registers before the buffer is refilled
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        asm volatile("" ::: "memory");
+        if (p + NB < n) load(p + NB);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+            if (kk == 0 || 64 * q + 32 < K) {  // K is a multiple of 32
+#pragma unroll
+                for (int i = 0; i < RB; ++i)
+#pragma unroll
+                    for (int j = 0; j < CB; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[kk][i], f[kk][RB + j], acc[i][j], 0, 0, 0);
+            }
+    }
+    hx_f4* part = reinterpret_cast<hx_f4*>(buf);  // [KS / 2][RB * CB][64]
+    __syncthreads();                              // every wave is done with its buffers
+#pragma unroll
+    for (int h = KS / 2; h >= 1; h >>= 1) {
+        if (wave >= h && wave < 2 * h) {
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int j = 0; j < CB; ++j) part[((wave - h) * RB * CB + i * CB + j) * 64 + lane] = acc[i][j];
         }
+        __syncthreads();
+        if (wave < h) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < RB; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < CB; ++j) acc[i][j] += part[(wave * RB * CB + i * CB + j) * 64 + lane];
+        }
+        if (h > 1) __syncthreads();
     }
+    if (wave != 0) return;
     // C: lane holds column lane % 16, rows 4 * (lane / 16) + r of each 16 x 16 block
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < RB; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < CB; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int m = r0 + 16 * i + 4 * (lane >> 4) + r, n = c0 + 16 * j + lr;
+                const int m = r0 + 16 * i + 4 * (lane >> 4) + r, n = c0 + 16 * j + (lane & 15);
                 if (m < M && n < N) store_out(y, (size_t)m * N + n, acc[i][j][r], y_fp32, add);
             }
+}
+
+template <int RB, int CB, int KS, int NB>
+__global__ __launch_bounds__(64 * KS) void gemm_nt_split_kernel(const _Float16* x, const _Float16* w, void* y, int M,
+                                                                int N, int K, bool y_fp32, bool add)
+{
+    gemm_nt_split<RB, CB, KS, NB>(x, w, y, M, N, K, y_fp32, add);
+}
+
+struct NtCall {
+    const _Float16 *x, *w;
+    void* y;
+    int M, N, K;
+    bool y_fp32, add;
+};
+
+// Rounds of workgroups (one per CU, by LDS) times the rows of x and w that a workgroup reads.
+template <int RB, int CB>
+static long nt_cost(const NtCall& c)
+{
+    const long wgs = (long)((c.M + 16 * RB - 1) / (16 * RB)) * ((c.N + 16 * CB - 1) / (16 * CB));
+    return (wgs + 255) / 256 * (RB + CB);
+}
+
+template <int RB, int CB, int KS, int NB>
+static hipError_t nt_launch(const NtCall& c, hipStream_t st)
+{
+    constexpr size_t lds = sizeof(_Float16) * KS * NB * 16 * (RB + CB) * 64;
+    hipLaunchKernelGGL((gemm_nt_split_kernel<RB, CB, KS, NB>),
+                       dim3((c.M + 16 * RB - 1) / (16 * RB), (c.N + 16 * CB - 1) / (16 * CB)), dim3(64 * KS), lds, st,
+                       c.x, c.w, c.y, c.M, c.N, c.K, c.y_fp32, c.add);
+    return hipGetLastError();
 }
 
 hipError_t launch_gemm_nt_f16(const _Float16* x, const _Float16* w, void* y, int M, int N, int K, bool y_fp32,
@@ -128,8 +224,20 @@ hipError_t launch_gemm_nt_f16(const _Float16* x, const _Float16* w, void* y, int
         else
             hipLaunchKernelGGL((gemv_nt_kernel<8>), dim3(N), dim3(256), 0, st, x, w, y, M, N, K, y_fp32, add);
     } else {
-        hipLaunchKernelGGL(gemm_nt_mfma_kernel, dim3((M + 127) / 128, (N + 31) / 32), dim3(256), 0, st, x, w, y, M,
-                           N, K, y_fp32, add);
+        // The tile with the least reading on the busiest CU; equal costs go to the larger tile (fewer bytes
+        // in all).
+        const NtCall c{x, w, y, M, N, K, y_fp32, add};
+        const long cost[5] = {nt_cost<4, 6>(c), nt_cost<4, 4>(c), nt_cost<2, 3>(c), nt_cost<2, 2>(c), nt_cost<1, 1>(c)};
+        int best = 0;
+        for (int i = 1; i < 5; ++i)
+            if (cost[i] < cost[best]) best = i;
+        switch (best) {
+            case 0: return nt_launch<4, 6, 4, 2>(c, st);
+            case 1: return nt_launch<4, 4, 4, 2>(c, st);
+            case 2: return nt_launch<2, 3, 8, 2>(c, st);
+            case 3: return nt_launch<2, 2, 8, 2>(c, st);
+            default: return nt_launch<1, 1, 16, 2>(c, st);
+        }
     }
     return hipGetLastError();
 }

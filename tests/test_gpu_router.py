@@ -115,3 +115,23 @@ def test_routing_ds3_nogroup_hidden(torch_mod, bias, act):
     exl3.routing_gemv(torch.from_numpy(x).cuda(), torch.from_numpy(gate).cuda(), s2, k, E)
     torch.cuda.synchronize()
     assert torch.equal(s2, scores)
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 1, 32), (17, 64, 96), (130, 160, 2016), (300, 96, 4096), (700, 130, 1056),
+                                   (1030, 288, 4064), (2049, 64, 128), (4100, 288, 512)])
+@pytest.mark.parametrize("add", [False, True])
+def test_gemm_nt_split_tiles(M, N, K, add):
+    """Every tile of the M > 8 kernel: remainders of rows, columns and k (a last chunk of 32), waves without
+    a k range.  The outputs have standard deviation sqrt(K); an fp32 sum of K such terms is off by at most
+    about K^0.5 * 2^-24 of that in a random walk (4e-6 at K = 4096), the largest of 1e6 outputs 5 times it."""
+    import torch
+    from helios_glm53flash_amd import exl3
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=g, device="cuda").half()
+    w = torch.randn((N, K), generator=g, device="cuda").half()
+    y = torch.randn((M, N), generator=g, device="cuda")
+    ref = x.double() @ w.double().T + (y.double() if add else 0.0)
+    exl3.gemm_nt_f16(y, x, w, M, N, K, y_fp32=True, add=add)
+    torch.cuda.synchronize()
+    assert float((y.double() - ref).abs().max()) <= 1e-5 * K ** 0.5 * 5
