@@ -614,8 +614,9 @@ __device__ __forceinline__ void down_epilogue(const MoeDecodeArgs& a, const Deco
         d0 = d0 * wgt * (float)sd.x;
         d1 = d1 * wgt * (float)sd.y;
         float* dst = a.contrib + row * a.hidden + c;
-        __hip_atomic_store(dst, d0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(dst + 1, d1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(reinterpret_cast<uint64_t*>(dst),
+                           (uint64_t)__float_as_uint(d0) | ((uint64_t)__float_as_uint(d1) << 32), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -624,32 +625,36 @@ __device__ __forceinline__ void down_epilogue(const MoeDecodeArgs& a, const Deco
 __device__ __forceinline__ void combine_columns(const MoeDecodeArgs& a, const DecodePlan& p, int cg, bool has_shared)
 {
     const int R = a.T * a.topk;
-    for (int i = threadIdx.x; i < a.T * 128; i += hx_nthreads()) {
-        const int t = i >> 7;
-        const int c = cg * 128 + (i & 127);
+    const __amdgpu_buffer_rsrc_t rc = coherent_rsrc(a.contrib);
+    for (int i = threadIdx.x; i < a.T * 32; i += hx_nthreads()) {
+        const int t = i >> 5, c = cg * 128 + 4 * (i & 31);
         // the loads of 8 contributions (and the shared row) are issued together, then added in
         // routing-rank order
         constexpr int B = 8;
-        float acc = 0.0f;
+        hx_f4 acc = {0.f, 0.f, 0.f, 0.f}, sh = {0.f, 0.f, 0.f, 0.f};
+        if (has_shared) sh = coherent_load4(rc, ((R + t) * a.hidden + c) * 4);
         for (int j0 = 0; j0 < a.topk; j0 += B) {
-            float v[B];
+            hx_f4 v[B];
 #pragma unroll
             for (int j = 0; j < B; ++j)
-                v[j] = __hip_atomic_load(a.contrib + (size_t)p.r2s[t * a.topk + min(j0 + j, a.topk - 1)] * a.hidden + c,
-                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                v[j] = coherent_load4(rc, (p.r2s[t * a.topk + min(j0 + j, a.topk - 1)] * a.hidden + c) * 4);
 #pragma unroll
             for (int j = 0; j < B; ++j)
                 if (j0 + j < a.topk) acc += v[j];
         }
-        const float sh = has_shared ? __hip_atomic_load(a.contrib + (size_t)(R + t) * a.hidden + c, __ATOMIC_RELAXED,
-                                                        __HIP_MEMORY_SCOPE_AGENT)
-                                    : 0.0f;
         const size_t o = (size_t)t * a.hidden + c;
-        if (a.y_routed) a.y_routed[o] = a.y_accumulate ? a.y_routed[o] + acc : acc;
+        if (a.y_routed) {
+            hx_f4u* yr = reinterpret_cast<hx_f4u*>(a.y_routed + o);
+            *yr = a.y_accumulate ? *yr + acc : acc;
+        }
         if (has_shared) acc += sh;
-        if (a.y) a.y[o] = (_Float16)acc;
+        if (a.y) {
+            typedef _Float16 h4u __attribute__((ext_vector_type(4), aligned(4)));
+            *reinterpret_cast<h4u*>(a.y + o) = h4u{(_Float16)acc[0], (_Float16)acc[1], (_Float16)acc[2], (_Float16)acc[3]};
+        }
     }
 }
+
 
 
 // ------------------------------------------------------------------ the layer kernel
@@ -766,39 +771,39 @@ __device__ __forceinline__ void gu_finish(const MoeDecodeArgs& a, const DecodePl
     const int ng = sp.count(cgate), nu = sp.count(cup);
     if (!arrive_last(&a.counter_gu[slot * gg + cg], ng + nu)) return;
     // the epilogue's scale pairs and both projections' partial sums in one round trip: the scale
-    // loads go first, the gate and up sums are gathered side by side (with one row, threads 0-127
-    // take the gate's columns and 128-255 the up's); the gate's svh of a non-gated expert need not
-    // exist
+    // loads go first, the gate and up sums are gathered side by side; the gate's svh of a non-gated
+    // expert need not exist
     const int lane = threadIdx.x & 63;
     const int col = cg * 128 + 2 * lane;
     auto ep = [&](int q) { return *reinterpret_cast<const hx_h2*>(static_cast<const _Float16*>(plan.tab.ep[q]) + col); };
     const hx_h2 sg = si.expert < 0 || a.act_fn != HX_ACT_RELU2_NOGATE ? ep(0) : hx_h2{(_Float16)0.0f, (_Float16)0.0f};
     const hx_h2 su = ep(1), sd = ep(2);
-    const float* pg = a.partial_g + (size_t)(slot * gg + cg) * (KB + 1) * 8 * 128;
-    const float* pu = a.partial_u + (size_t)(slot * gg + cg) * (KB + 1) * 8 * 128;
-    for (int i = threadIdx.x; i < 2 * MT * 128; i += hx_nthreads()) {
-        const bool up = i >= MT * 128;
-        const int k = up ? i - MT * 128 : i, m = k >> 7;
-        const int n = up ? nu : ng;
-        float v = 0.0f;
-        if (m < si.count && (up || gated)) {
-            // segment s, row m of the partial sums: (s * rows + m) * 128 + column; 8 segments' loads
-            // together, added in segment order
-            const float* p = (up ? pu : pg) + (size_t)m * 128 + (k & 127);
-            const size_t stride = (size_t)si.count * 128;
-            constexpr int B = 8;
-            for (int s0 = 0; s0 < n; s0 += B) {
-                float t[B];
+    // a thread takes 4 columns of a row; segment i, row m of the partial sums: (i * rows + m) * 128 + column;
+    // 8 segments' loads together, added in segment order
+    const int rows = si.count, half = min(rows, MT) * 32;
+    const __amdgpu_buffer_rsrc_t rg = coherent_rsrc(a.partial_g + (size_t)(slot * gg + cg) * (KB + 1) * 8 * 128);
+    const __amdgpu_buffer_rsrc_t ru = coherent_rsrc(a.partial_u + (size_t)(slot * gg + cg) * (KB + 1) * 8 * 128);
+    auto sum = [&](__amdgpu_buffer_rsrc_t r, int k, int n, float* out) {
+        hx_f4 v = {0.f, 0.f, 0.f, 0.f};
+        constexpr int B = 8;
+        for (int s0 = 0; s0 < n; s0 += B) {
+            hx_f4 t[B];
 #pragma unroll
-                for (int j = 0; j < B; ++j)
-                    t[j] = __hip_atomic_load(p + (size_t)min(s0 + j, n - 1) * stride, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT);
+            for (int j = 0; j < B; ++j) t[j] = coherent_load4(r, (min(s0 + j, n - 1) * rows * 32 + k) * 16);
 #pragma unroll
-                for (int j = 0; j < B; ++j)
-                    if (s0 + j < n) v += t[j];
-            }
+            for (int j = 0; j < B; ++j)
+                if (s0 + j < n) v += t[j];
         }
-        (up ? cs_u : cs_g)[k] = v;
+        *reinterpret_cast<hx_f4*>(out + 4 * k) = v;
+    };
+    // up to 4 rows: the gate's pieces on waves 0 and 1, the up's on 2 and 3, at the same time
+    const bool both = half <= 128;
+    for (int i = threadIdx.x; i < (both ? 256 : 2 * half); i += hx_nthreads()) {
+        const bool up = both ? i >= 128 : i >= half;
+        const int k = up ? i - (both ? 128 : half) : i;
+        if (k >= half) continue;
+        if (up) sum(ru, k, nu, cs_u);
+        else if (gated) sum(rg, k, ng, cs_g);
     }
     __syncthreads();
     guad_epilogue<MT>(a, plan, si, slot, cg, cs_g, cs_u, sg, su, sd);
