@@ -37,10 +37,8 @@ HIP_FLAGS = [
 # selection the accumulators live in AGPRs while the MFMAs are selected in their VGPR form, and every
 # k step copies them back and forth (3 extra VALU moves per MFMA on gfx950, measured in the
 # generated code).
-FILE_FLAGS = {
-    "hx_moe_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
-    "hx_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
-}
+_VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
+FILE_FLAGS = {f: _VGPR_FORM for f in ("hx_moe_prefill.hip", "hx_gemm.hip", *(f"hx_gemm_b{b}.hip" for b in range(1, 9)))}
 
 
 def _compile(src: Path) -> Path:

@@ -173,11 +173,20 @@ static int decode_checked(int r, void* workspace, hx_stream_t stream)
     return hx_moe_check_status(workspace, stream);
 }
 
-size_t hx_exl3_gemm_workspace_size(int M, int N, int K)
+// What a call needs at least (M > 16: nothing but the transformed input, when a_had is null).
+static size_t gemm_min_bytes(int M, int N, int K)
 {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     if (M <= hx::GEMV_MAX_M) return hx::gemv_workspace_bytes(M, K, N);
     return hx::HX_COUNTER_BYTES + align256((size_t)M * K * sizeof(_Float16));
+}
+
+size_t hx_exl3_gemm_workspace_size(int M, int N, int K)
+{
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    const size_t least = gemm_min_bytes(M, N, K);
+    if (M <= hx::GEMV_MAX_M) return least;
+    return least + hx::mfma_rs_bytes(M, K) + hx::mfma_partial_bytes(M, K, N);
 }
 
 int hx_exl3_gemm(void* y, const void* x, const hx_group_words* w, int M, int N, int K, int bits, int y_fp32,
@@ -208,9 +217,22 @@ int hx_exl3_gemm(void* y, const void* x, const hx_group_words* w, int M, int N, 
             return fail(HX_ERR_WORKSPACE, "hx_exl3_gemm: a_had is null and the workspace cannot hold M*K fp16");
         ah = reinterpret_cast<_Float16*>(static_cast<char*>(workspace) + hx::HX_COUNTER_BYTES);
     }
-    int r = hip_status(hx::launch_input_had(xh, suh, ah, M, K, st), "hx_exl3_gemm(input transform)");
+    // row sums of the transformed input and K-split partials go to what the workspace has beyond the
+    // counters and (a_had null) the transformed input; a smaller workspace does without them
+    float* rs = nullptr;
+    void* partial = nullptr;
+    size_t o = hx::HX_COUNTER_BYTES + (a_had ? 0 : align256((size_t)M * K * sizeof(_Float16)));
+    if (workspace && workspace_bytes >= o + hx::mfma_rs_bytes(M, K)) {
+        rs = reinterpret_cast<float*>(static_cast<char*>(workspace) + o);
+        o += hx::mfma_rs_bytes(M, K);
+        const size_t pb = hx::mfma_partial_bytes(M, K, N);
+        if (pb && workspace_bytes >= o + pb) partial = static_cast<char*>(workspace) + o;
+    }
+    int r = hip_status(hx::launch_input_had(xh, suh, ah, rs, M, K, st), "hx_exl3_gemm(input transform)");
     if (r) return r;
-    r = hip_status(hx::launch_linear_mfma(ah, tr, svh, y, M, K, N, bits, cb, y_fp32 != 0, st), "hx_exl3_gemm(mfma)");
+    r = hip_status(hx::launch_linear_mfma(ah, rs, tr, svh, y, M, K, N, bits, cb, y_fp32 != 0, partial,
+                                          static_cast<int*>(workspace), st),
+                   "hx_exl3_gemm(mfma)");
     return r ? r : HX_GEMM_PATH_MFMA;
 }
 
@@ -260,7 +282,7 @@ int hx_exl3_gemm_noalloc(void* y, const void* x, const hx_group_words* w, int M,
                          hx_stream_t stream, int mcg)
 {
     if (M < 0 || N <= 0 || K <= 0) return fail(HX_ERR_INVALID, "hx_exl3_gemm_noalloc: bad extents");
-    const size_t need = hx_exl3_gemm_workspace_size(M, N, K);
+    const size_t need = gemm_min_bytes(M, N, K);
     if (need > HX_NOALLOC_SCRATCH_BYTES) {
         snprintf(g_err, sizeof(g_err),
                  "hx_exl3_gemm_noalloc: M=%d N=%d K=%d needs %zu bytes of scratch, more than its %zu (use hx_exl3_gemm "
@@ -695,16 +717,16 @@ int hx_moe_layer(void* y, float* y_routed, const void* x, const void* scores, co
         float* sh_d = reinterpret_cast<float*>(base + L.off_sh_d);
         auto H = [](const void* p) { return static_cast<const _Float16*>(p); };
         auto U16 = [](const void* p) { return static_cast<const uint16_t*>(p); };
-        hipError_t e = hx::launch_input_had(xh, H(shared[0].suh), sh_a, tokens, hidden_dim, st);
-        if (!e) e = hx::launch_linear_mfma(sh_a, U16(shared[0].trellis), H(shared[0].svh), sh_g, tokens, hidden_dim,
-                                           intermediate_dim, shared_bits[0], cb, true, st);
-        if (!e) e = hx::launch_input_had(xh, H(shared[1].suh), sh_a, tokens, hidden_dim, st);
-        if (!e) e = hx::launch_linear_mfma(sh_a, U16(shared[1].trellis), H(shared[1].svh), sh_u, tokens, hidden_dim,
-                                           intermediate_dim, shared_bits[1], cb, true, st);
+        hipError_t e = hx::launch_input_had(xh, H(shared[0].suh), sh_a, nullptr, tokens, hidden_dim, st);
+        if (!e) e = hx::launch_linear_mfma(sh_a, nullptr, U16(shared[0].trellis), H(shared[0].svh), sh_g, tokens, hidden_dim,
+                                           intermediate_dim, shared_bits[0], cb, true, nullptr, nullptr, st);
+        if (!e) e = hx::launch_input_had(xh, H(shared[1].suh), sh_a, nullptr, tokens, hidden_dim, st);
+        if (!e) e = hx::launch_linear_mfma(sh_a, nullptr, U16(shared[1].trellis), H(shared[1].svh), sh_u, tokens, hidden_dim,
+                                           intermediate_dim, shared_bits[1], cb, true, nullptr, nullptr, st);
         if (!e) e = hx::launch_swiglu_clamp(sh_g, sh_u, sh_act, (size_t)tokens * intermediate_dim, act_limit, st);
-        if (!e) e = hx::launch_input_had(sh_act, H(shared[2].suh), sh_a, tokens, intermediate_dim, st);
-        if (!e) e = hx::launch_linear_mfma(sh_a, U16(shared[2].trellis), H(shared[2].svh), sh_d, tokens,
-                                           intermediate_dim, hidden_dim, shared_bits[2], cb, true, st);
+        if (!e) e = hx::launch_input_had(sh_act, H(shared[2].suh), sh_a, nullptr, tokens, intermediate_dim, st);
+        if (!e) e = hx::launch_linear_mfma(sh_a, nullptr, U16(shared[2].trellis), H(shared[2].svh), sh_d, tokens,
+                                           intermediate_dim, hidden_dim, shared_bits[2], cb, true, nullptr, nullptr, st);
         if ((r = hip_status(e, "hx_moe_layer(shared expert)"))) return r;
         shared_rows = sh_d;
     }

@@ -1,109 +1,106 @@
-// hx_gemm.hip -- EXL3 quantized linear for M > 8 on MFMA (gfx950): input transform kernel, then
-// quarter-operand MFMA tiles (hx_mfma.hpp) with the output Hadamard + svh epilogue fused.
-// Reference semantics: src/cuda/quant/exl3_gemm_kernel.cuh:8-80, exl3_gemm_inner.cuh:456-480.
-#include "hx_mfma.hpp"
-#include "hx_kernels.hpp"
+// hx_gemm.hip -- EXL3 quantized linear for M > 16 on MFMA (gfx950): the input transform kernel, the plan and
+// the dispatch (tile kernels in hx_gemm_impl.hpp, one translation unit per bit width: hx_gemm_b<bits>.hip).
+#include "hx_gemm_impl.hpp"
 
 namespace hx {
 
-// a = fp16(H128(fp16(x . suh))) row-wise (had_hf_r_128_inner<true,false>); one wave per 128 block.
-__global__ __launch_bounds__(256) void input_had_kernel(const _Float16* x, const _Float16* suh, _Float16* a,
-                                                        long blocks, int K)
-{
-    const int lane = threadIdx.x & 63;
-    const long b = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (b >= blocks) return;
-    const long row = b / (K / 128);
-    const int c = (int)(b % (K / 128)) * 128 + 2 * lane;
-    hx_h2 v = *reinterpret_cast<const hx_h2*>(x + row * K + c) * *reinterpret_cast<const hx_h2*>(suh + c);
-    float v0 = (float)v.x, v1 = (float)v.y;
-    hx_had128_wave(v0, v1);
-    hx_h2 o = {(_Float16)v0, (_Float16)v1};
-    *reinterpret_cast<hx_h2*>(a + row * K + c) = o;
-}
+template <int BITS>
+hipError_t launch_mfma_b(int cb, const MfmaGemmArgs& g, hipStream_t st);  // hx_gemm_b*.hip
 
-hipError_t launch_input_had(const _Float16* x, const _Float16* suh, _Float16* a, long rows, int K, hipStream_t st)
+// a = fp16(H128(fp16(x . suh))) row-wise (had_hf_r_128_inner<true,false>) and, with rs, the fp32 sum of each
+// 128-wide block of a.  One wave per 16 consecutive blocks on the matrix cores (hx_gemv.hpp), the
+// results stored 16 bytes per lane through LDS.  Bound: memory; M = 2000, K = 4096 (33 MB) 15.6 us with
+// one block per wave and a shuffle butterfly.
+constexpr int HAD_LD = 128 + 8;  // halves per staged block
+__global__ __launch_bounds__(256) void input_had_kernel(const _Float16* x, const _Float16* suh, _Float16* a, float* rs,
+                                                        long blocks, int nblk)
 {
-    long blocks = rows * (K / 128);
-    if (blocks == 0) return hipSuccess;
-    hipLaunchKernelGGL(input_had_kernel, dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, st, x, suh, a, blocks, K);
-    return hipGetLastError();
-}
-
-// Output epilogue for a staged 64-row half: y[row][cg*128 + c] = svh . H128(C[row][:]).
-template <int CB, class Smem>
-__device__ void linear_tile_epilogue(const Smem& sm, int half, int rows, const _Float16* svh, void* y, int N,
-                                     int cg, bool y_fp32)
-{
+    __shared__ _Float16 stage[4][16 * HAD_LD];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int c = cg * 128 + 2 * lane;
-    const hx_h2 sv = *reinterpret_cast<const hx_h2*>(svh + c);
-    for (int r = wave; r < 64; r += 4) {
-        const int row = 64 * half + r;
-        if (row >= rows) break;
-        float v0 = staged_value<CB>(sm, half, r, 2 * lane), v1 = staged_value<CB>(sm, half, r, 2 * lane + 1);
-        hx_had128_wave(v0, v1);
-        if (y_fp32) {
-            *reinterpret_cast<float2*>(static_cast<float*>(y) + (size_t)row * N + c) =
-                make_float2(v0 * (float)sv.x, v1 * (float)sv.y);
-        } else {
-            hx_h2 h = {(_Float16)v0, (_Float16)v1};
-            *reinterpret_cast<hx_h2*>(static_cast<_Float16*>(y) + (size_t)row * N + c) = h * sv;
+    const long b0 = ((long)blockIdx.x * 4 + wave) * 16;
+    if (b0 >= blocks) return;
+    const int g = lane >> 4;
+    const long b = min(b0 + (lane & 15), blocks - 1);
+    const _Float16* xb = x + b * 128 + 8 * g;
+    const _Float16* sb = suh + (b % nblk) * 128 + 8 * g;
+    InputRegs r;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+        r.x[kk] = *reinterpret_cast<const hx_h8u*>(xb + 32 * kk);
+        r.s[kk] = *reinterpret_cast<const hx_h8u*>(sb + 32 * kk);
+    }
+    _Float16* sw = stage[wave];
+    input_store(reinterpret_cast<uint32_t*>(sw), r, 16, 0, HAD_LD);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int j = 4 * q + g, c8 = 8 * (lane & 15);
+        const hx_h8 v = *reinterpret_cast<const hx_h8*>(sw + j * HAD_LD + c8);
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s += (float)v[i];
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 64);
+        if (b0 + j < blocks) {
+            *reinterpret_cast<hx_h8u*>(a + (b0 + j) * 128 + c8) = v;
+            if (rs && (lane & 15) == 0) rs[b0 + j] = s;
         }
     }
 }
 
-// Quarter-operand tile (each wave decodes its own 32 columns into MFMA B operands; only A is staged
-// in LDS), three workgroups per CU.
-template <int BITS, int CB>
-__global__ __launch_bounds__(MF_THREADS, qt_occ<CB>()) void linear_mfma_kernel(const _Float16* a, const uint32_t* trellis,
-                                                                const _Float16* svh, void* y, int M, int K, int N,
-                                                                bool y_fp32)
+hipError_t launch_input_had(const _Float16* x, const _Float16* suh, _Float16* a, float* rs, long rows, int K,
+                            hipStream_t st)
 {
-    __shared__ MfmaSmemQ sm;
-    // the row tiles of a column group on one XCD: its trellis words come from memory once and the
-    // other row tiles read them from that XCD's L2
-    int mt, cg;
-    xcd_group_index(blockIdx.x + blockIdx.y * gridDim.x, gridDim.y, gridDim.x, mt, cg);
-    const int m0 = mt * MF_BM;
-    const int rows = min(MF_BM, M - m0);
-    hx_f4 acc[MF_BM / 16][2];
-    mfma_tile_q<BITS, CB, MF_BM>(a + (size_t)m0 * K, K, rows, trellis, K, N, cg * 8, sm, acc);
-    void* yt = y_fp32 ? (void*)(static_cast<float*>(y) + (size_t)m0 * N) : (void*)(static_cast<_Float16*>(y) + (size_t)m0 * N);
-    for (int half = 0; half < 2; ++half) {
-        qt_stage_c_half<MF_BM>(acc, half, sm);
-        __syncthreads();
-        linear_tile_epilogue<CB>(sm, half, rows, svh, yt, N, cg, y_fp32);
-        __syncthreads();
-    }
-}
-
-template <int BITS>
-static hipError_t launch_mfma_b(int cb, const _Float16* a, const uint32_t* tr, const _Float16* svh, void* y, int M,
-                                int K, int N, bool y_fp32, hipStream_t st)
-{
-    dim3 grid(N / 128, (M + MF_BM - 1) / MF_BM);
-    switch (cb) {
-        case 0: hipLaunchKernelGGL((linear_mfma_kernel<BITS, 0>), grid, dim3(MF_THREADS), 0, st, a, tr, svh, y, M, K, N, y_fp32); break;
-        case 1: hipLaunchKernelGGL((linear_mfma_kernel<BITS, 1>), grid, dim3(MF_THREADS), 0, st, a, tr, svh, y, M, K, N, y_fp32); break;
-        default: hipLaunchKernelGGL((linear_mfma_kernel<BITS, 2>), grid, dim3(MF_THREADS), 0, st, a, tr, svh, y, M, K, N, y_fp32); break;
-    }
+    const long blocks = rows * (K / 128);
+    if (blocks == 0) return hipSuccess;
+    hipLaunchKernelGGL(input_had_kernel, dim3((unsigned)((blocks + 63) / 64)), dim3(256), 0, st, x, suh, a, rs, blocks,
+                       K / 128);
     return hipGetLastError();
 }
 
-hipError_t launch_linear_mfma(const _Float16* a_had, const uint16_t* trellis, const _Float16* svh, void* y, int M,
-                              int K, int N, int bits, int cb, bool y_fp32, hipStream_t st)
+// K splits: tiles that leave more than half of the 768 resident workgroups (3 on each of 256 CUs) empty are split,
+// with at least 8 chunks of 64 k each.  A split costs its accumulators a trip through memory (written, then
+// read by the last to arrive), so past 5 splits only up to 2 workgroups per CU.  4096 -> 12288 4-bit (96 row x
+// column tiles) at M = 45 / 128: 58 / 67 us unsplit, 35.0 / 49.4 with 2, 28.8 / 42.6 with 4, 27.3 / 41.1 with 5,
+// 28.9 / 49.4 with 8; 24576 columns (192 tiles) at M = 45: 44.6 with 2, 36.5 with 4; 8192 -> 8192 (64 tiles): 63.0
+// with 2, 42.3 with 5, 37.1 with 8 (graphs of 10 calls, input transform included).
+int mfma_splits(int M, int K, int N)
 {
-    const uint32_t* tr = reinterpret_cast<const uint32_t*>(trellis);
+    const long tiles = (long)((M + MF_BM - 1) / MF_BM) * (N / 128), nk = K / MF_BK;
+    auto least = [](long a, long b) { return a < b ? a : b; };
+    const long two = 2 * GEMV_CUS / tiles;
+    const long s = least(least(3 * GEMV_CUS / tiles, two > 5 ? two : 5), least(nk / 8, 8));
+    return s > 1 ? (int)s : 1;
+}
+
+static size_t al256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+size_t mfma_rs_bytes(int M, int K) { return al256((size_t)M * (K / 128) * sizeof(float)); }
+
+size_t mfma_partial_bytes(int M, int K, int N)
+{
+    const int s = mfma_splits(M, K, N);
+    if (s == 1) return 0;
+    return (size_t)((M + MF_BM - 1) / MF_BM) * (N / 128) * s * MF_BM * 128 * sizeof(float);
+}
+
+hipError_t launch_linear_mfma(const _Float16* a_had, const float* rs, const uint16_t* trellis, const _Float16* svh,
+                              void* y, int M, int K, int N, int bits, int cb, bool y_fp32, void* partial, int* counter,
+                              hipStream_t st)
+{
+    MfmaGemmArgs g{a_had, rs, reinterpret_cast<const uint32_t*>(trellis), svh, y, M, K, N, y_fp32,
+                   rs && partial ? mfma_splits(M, K, N) : 1, static_cast<hx_f4*>(partial), counter};
     switch (bits) {
-        case 1: return launch_mfma_b<1>(cb, a_had, tr, svh, y, M, K, N, y_fp32, st);
-        case 2: return launch_mfma_b<2>(cb, a_had, tr, svh, y, M, K, N, y_fp32, st);
-        case 3: return launch_mfma_b<3>(cb, a_had, tr, svh, y, M, K, N, y_fp32, st);
-        case 4: return launch_mfma_b<4>(cb, a_had, tr, svh, y, M, K, N, y_fp32, st);
-        case 5: return launch_mfma_b<5>(cb, a_had, tr, svh, y, M, K, N, y_fp32, st);
-        case 6: return launch_mfma_b<6>(cb, a_had, tr, svh, y, M, K, N, y_fp32, st);
-        case 7: return launch_mfma_b<7>(cb, a_had, tr, svh, y, M, K, N, y_fp32, st);
-        case 8: return launch_mfma_b<8>(cb, a_had, tr, svh, y, M, K, N, y_fp32, st);
+        case 1: return launch_mfma_b<1>(cb, g, st);
+        case 2: return launch_mfma_b<2>(cb, g, st);
+        case 3: return launch_mfma_b<3>(cb, g, st);
+        case 4: return launch_mfma_b<4>(cb, g, st);
+        case 5: return launch_mfma_b<5>(cb, g, st);
+        case 6: return launch_mfma_b<6>(cb, g, st);
+        case 7: return launch_mfma_b<7>(cb, g, st);
+        case 8: return launch_mfma_b<8>(cb, g, st);
         default: return hipErrorInvalidValue;
     }
 }

@@ -1,0 +1,6 @@
+// Instantiation of the MFMA linear kernels for 5-bit trellis.
+#include "hx_gemm_impl.hpp"
+
+namespace hx {
+template hipError_t launch_mfma_b<5>(int, const MfmaGemmArgs&, hipStream_t);
+}  // namespace hx

@@ -28,9 +28,17 @@ hipError_t launch_linear_gemv(const _Float16* x, const uint16_t* trellis, const 
                               void* y, int M, int K, int N, int bits, int cb, bool y_fp32, void* ws, hipStream_t st);
 
 // large-M linear on MFMA (hx_gemm.hip)
-hipError_t launch_input_had(const _Float16* x, const _Float16* suh, _Float16* a, long rows, int K, hipStream_t st);
-hipError_t launch_linear_mfma(const _Float16* a_had, const uint16_t* trellis, const _Float16* svh, void* y,
-                              int M, int K, int N, int bits, int cb, bool y_fp32, hipStream_t st);
+// rs: optional [rows][K / 128] fp32 sums of the transformed blocks (mfma_rs_bytes).
+hipError_t launch_input_had(const _Float16* x, const _Float16* suh, _Float16* a, float* rs, long rows, int K,
+                            hipStream_t st);
+// rs (null: slower tiles that sum the input themselves), partial and counter (null: no K splits) are
+// workspace: mfma_partial_bytes, and zeroed arrival counters that are left at zero.
+hipError_t launch_linear_mfma(const _Float16* a_had, const float* rs, const uint16_t* trellis, const _Float16* svh,
+                              void* y, int M, int K, int N, int bits, int cb, bool y_fp32, void* partial, int* counter,
+                              hipStream_t st);
+int mfma_splits(int M, int K, int N);
+size_t mfma_rs_bytes(int M, int K);
+size_t mfma_partial_bytes(int M, int K, int N);
 
 // utilities (hx_misc.hip)
 hipError_t launch_reconstruct(_Float16* out, const uint16_t* packed, int packed_rows, int packed_cols,

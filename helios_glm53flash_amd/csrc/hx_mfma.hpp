@@ -73,10 +73,10 @@ HX_INLINE void qt_rowcol(int rb, int nh, int i, int& row, int& col)
     col = 32 * wave + 16 * ((lane >> 3) & 1) + 8 * nh + (lane & 7);
 }
 
-// Chunks of global loads in flight for the quarter-operand tile (2 keeps it at 3 workgroups per CU):
-// A chunks (QT_PF) and trellis-word chunks (QT_PT).
+// Chunks of global loads in flight for the quarter-operand tile, of A and of trellis words: 2 at 96 and 128
+// rows (more would cost the 3 workgroups per CU), 4 at 32 and 64 rows, whose A buffers are smaller.
 constexpr int QT_PF = 2;
-constexpr int QT_PT = 2;
+constexpr int qt_pf(int bm) { return bm <= 64 ? 4 : QT_PF; }
 // The next chunk's decode runs after the chunk's MFMAs.  (Slicing it between the row blocks' MFMAs,
 // so that one wave overlaps its own VALU and matrix work, measured equal on the config-4 prefill:
 // 3.14 ms either way; the co-resident waves of a SIMD already overlap the two.)
@@ -88,7 +88,7 @@ constexpr int QT_PT = 2;
 constexpr int QT_OCC = 3;
 template <int CB>
 constexpr int qt_occ() { return CB == 2 ? QT_OCC : 2; }
-// LDS A buffers: with A loaded straight into LDS, the chunks in flight and the one being read
+// LDS A buffers of 128 rows: with A loaded straight into LDS, the chunks in flight and the one being read
 constexpr int QT_NB = QT_PF + 1;
 // s_waitcnt immediate that waits until at most n vector-memory instructions are outstanding
 // (gfx9 encoding: vmcnt in bits 3:0 and 15:14; expcnt and lgkmcnt left at their no-wait maxima)
@@ -134,7 +134,7 @@ HX_INLINE bool xcd_group_index(int i, int nx, int ngroups, int& member, int& gro
 
 // With rs_src (codebook 2), the row sums of A come precomputed as rs_n fp32 partial sums per row
 // (rs_src[r * rs_n + b]) instead of being accumulated from the staged A.
-template <int BITS, int CB, int BM, int PF = QT_PF, bool EXT_RS = false, class Smem>
+template <int BITS, int CB, int BM, bool EXT_RS = false, int PFD = qt_pf(BM), class Smem>
 __device__ __forceinline__ void mfma_tile_q(const _Float16* A, long lda, int rows, const uint32_t* trellis, int K,
                                             int N, int tn0, Smem& sm, hx_f4 (&acc)[BM / 16][2],
                                             const float* rs_src = nullptr, int rs_n = 0)
@@ -163,10 +163,13 @@ __device__ __forceinline__ void mfma_tile_q(const _Float16* A, long lda, int row
 
     // A and the trellis words have rings of their own: PF chunks of A (16 VGPRs per chunk at BM 128),
     // PT chunks of trellis words (BITS + 1 VGPRs per chunk)
-    constexpr int PT = QT_PT;
     // A through LDS by DMA, unless the tile sums A's rows itself (that reads A in registers)
     constexpr bool DMA = EXT_RS || CB != 2;
-    static_assert(!DMA || (MF_LDA == MF_BK && PF + 1 <= QT_NB), "A ring in LDS");
+    constexpr int PF = DMA ? PFD : QT_PF, PT = PF;
+    constexpr int NB = DMA ? PF + 1 : 2;  // LDS A buffers
+    static_assert(MF_LDA == MF_BK && NB * BM <= QT_NB * MF_BM, "A ring in LDS");
+    _Float16* const ab = &sm.ab[0][0];
+    auto a_buf = [&](int b) { return ab + b * (BM * MF_LDA); };
     hx_u4v av[DMA ? 1 : PF][NA];
     uint32_t wv[PT][BITS + 1];
     float rs[NA];
@@ -195,11 +198,11 @@ __device__ __forceinline__ void mfma_tile_q(const _Float16* A, long lda, int row
 #pragma unroll
         for (int i = 0; i < NA; ++i)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                ra, (__attribute__((address_space(3))) void*)(&sm.ab[buf][(32 * i + 8 * wave_s) * MF_LDA]), 16,
+                ra, (__attribute__((address_space(3))) void*)(a_buf(buf) + (32 * i + 8 * wave_s) * MF_LDA), 16,
                 a_voff_lds[i], k0 * 2, 0, 0);
     };
     auto store_a = [&](int slot, int buf, bool count) {
-        _Float16* as = sm.ab[buf];
+        _Float16* as = a_buf(buf);
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
             const int idx = t + MF_THREADS * i;
@@ -261,10 +264,10 @@ __device__ __forceinline__ void mfma_tile_q(const _Float16* A, long lda, int row
     // step c: ua = c % PF, ut = c % PT, par = c & 1, all compile-time in the unrolled loops
     auto step = [&](int c, auto ua_, auto ut_, auto par_) {
         constexpr int ua = decltype(ua_)::value, ut = decltype(ut_)::value, par = decltype(par_)::value;
-        if constexpr (DMA) load_a_lds((c + PF) % QT_NB, min(c + PF, nk - 1) * MF_BK);
+        if constexpr (DMA) load_a_lds((c + PF) % NB, min(c + PF, nk - 1) * MF_BK);
         else load_a(ua, min(c + PF, nk - 1) * MF_BK);
         load_t(ut, min(c + PT, nk - 1) * MF_BK);
-        const _Float16* as = sm.ab[DMA ? c % QT_NB : c & 1];
+        const _Float16* as = a_buf(c % NB);
         const uint32_t* dc = d[par % ND];
         uint32_t* dn = d[(par + 1) % ND];
         const hx_h8 b00 = quarter_operand<0, 0>(dc), b01 = quarter_operand<0, 1>(dc);

@@ -222,7 +222,7 @@ __device__ __forceinline__ void grouped_tile(const GroupedGemmArgs& g, const Job
     const _Float16* A = g.A[proj] + (size_t)job.row0 * g.K;
     const uint32_t* tr = static_cast<const uint32_t*>(g.tr[proj][job.expert]);
     hx_f4 acc[BM / 16][2];
-    mfma_tile_q<BITS, CB, BM, QT_PF, true>(A, g.K, job.rows, tr, g.K, g.N, cg * 8, sm, acc,
+    mfma_tile_q<BITS, CB, BM, true, BM <= 32 ? 4 : QT_PF>(A, g.K, job.rows, tr, g.K, g.N, cg * 8, sm, acc,
                                             g.rs[proj] + (size_t)job.row0 * g.rs_n, g.rs_n);
     _Float16* out = g.out[proj] + (size_t)job.row0 * g.N + cg * 128;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -310,7 +310,7 @@ template <int BITS, int CB, int BM>
 __device__ __forceinline__ void gu_tile(const _Float16* A, int K, int rows, const void* tr, int N, int cg,
                                         GuSmem& sm, GuAcc<BM>& acc, const float* rs)
 {
-    mfma_tile_q<BITS, CB, BM, QT_PF, true>(A, K, rows, static_cast<const uint32_t*>(tr), K, N, cg * 8, sm, acc, rs,
+    mfma_tile_q<BITS, CB, BM, true, QT_PF>(A, K, rows, static_cast<const uint32_t*>(tr), K, N, cg * 8, sm, acc, rs,
                                            K / 128);
 }
 

@@ -118,6 +118,52 @@ def test_mfma_parity(hx, M, bits, cb):
     assert_close(got, ref, what=f"mfma M={M} bits={bits} cb={cb}")
 
 
+@pytest.mark.parametrize("M,K,N,bits,cb", [(17, 4096, 256, 4, 2), (32, 640, 128, 2, 2), (33, 1152, 384, 3, 0),
+                                           (64, 4096, 128, 5, 1), (65, 2176, 256, 8, 2), (97, 4096, 128, 2, 2),
+                                           (129, 1024, 256, 6, 2), (224, 3968, 128, 1, 2), (300, 512, 128, 7, 0)])
+@pytest.mark.parametrize("y_fp32", [False, True])
+def test_mfma_row_tiles_and_k_splits(hx, M, K, N, bits, cb, y_fp32):
+    """Row tiles of every height with full and partial rows; K split into unequal chunk counts, and too short
+    to split."""
+    for _ in range(2):  # the second call finds the arrival counters as the first left them
+        path, got, ref = _run_linear(hx, M, K, N, bits, cb, y_fp32, seed=M + K)
+        assert path == hx.HX_GEMM_PATH_MFMA
+        assert_close(got, ref, what=f"mfma M={M} K={K} N={N} bits={bits} cb={cb}")
+
+
+@pytest.mark.parametrize("ws_bytes", [0, 64 * 1024, 64 * 1024 + 45 * 8 * 4, None])
+def test_mfma_small_workspace(hx, ws_bytes):
+    """a_had given and no workspace, or one too small for the row sums or the K-split partials: the call does
+    without what does not fit."""
+    import ctypes as C
+    import torch
+    from oracle import oracle as O
+    from helios_glm53flash_amd._lib import lib
+    M, K, N, bits = 45, 1024, 256, 4
+    tr, suh, svh = make_linear(21, K, N, bits)
+    x = make_x(22, M, K)
+    w = hx.GroupWords(_dev(tr, torch.int16), _dev(suh), _dev(svh), hx.MUL1)
+    ref = O.linear(x, tr, suh, svh, K, N, bits, 2, out_f16=False)
+    xd, a_had, y = _dev(x), torch.empty((M, K), dtype=torch.float16, device="cuda"), torch.empty((M, N), device="cuda")
+    n = lib.hx_exl3_gemm_workspace_size(M, N, K) if ws_bytes is None else ws_bytes
+    ws = torch.zeros(n + 256, dtype=torch.uint8, device="cuda")
+    ws[n:] = 7
+    gw = w.c()
+    r = lib.hx_exl3_gemm(y.data_ptr(), xd.data_ptr(), C.byref(gw), M, N, K, bits, 1, None, a_had.data_ptr(), 0,
+                         ws.data_ptr() if n else None, n)
+    torch.cuda.synchronize()
+    assert r == hx.HX_GEMM_PATH_MFMA
+    assert_close(y.cpu().numpy(), ref, what=f"workspace {ws_bytes}")
+    assert bool((ws[n:] == 7).all()) and not bool(ws[:min(n, 64 * 1024)].any())
+
+
+def test_gemv_many_splits(hx):
+    """More K splits than the last arriver reads together, with 1 and 2 16-byte pieces per thread."""
+    for M in (3, 8, 11, 16):
+        _, got, ref = _run_linear(hx, M, 9 * 512, 128, 4, 2, False, seed=60 + M)
+        assert_close(got, ref, what=f"gemv splits M={M}")
+
+
 def test_mfma_fp16_out(hx):
     _, got, ref = _run_linear(hx, 64, 1024, 256, 2, 2, False, seed=77)
     assert_close(got, ref, what="mfma fp16")
