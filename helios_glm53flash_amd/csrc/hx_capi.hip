@@ -618,10 +618,10 @@ int hx_moe_grouped(const void* x, float* y, const int64_t* expert_count, const i
     p.lay = &L;
     if (sorted_contributions) {
         // contributions only: combine writes them; no y
-        return hip_status(hx::run_moe_prefill(p, sorted_contributions, nullptr, nullptr, nullptr, false, st),
+        return hip_status(hx::run_moe_prefill(p, sorted_contributions, nullptr, nullptr, false, st),
                           "hx_moe_grouped(prefill)");
     }
-    return hip_status(hx::run_moe_prefill(p, nullptr, nullptr, nullptr, y, true, st), "hx_moe_grouped(prefill)");
+    return hip_status(hx::run_moe_prefill(p, nullptr, nullptr, y, true, st), "hx_moe_grouped(prefill)");
 }
 
 int hx_moe_layer(void* y, float* y_routed, const void* x, const void* scores, const void* bias,
@@ -707,29 +707,6 @@ int hx_moe_layer(void* y, float* y_routed, const void* x, const void* scores, co
     }
     if (r) return r;
 
-    const float* shared_rows = nullptr;
-    if (shared) {
-        Phase ph(5, st);
-        _Float16* sh_a = reinterpret_cast<_Float16*>(base + L.off_sh_a);
-        float* sh_g = reinterpret_cast<float*>(base + L.off_sh_g);
-        float* sh_u = reinterpret_cast<float*>(base + L.off_sh_u);
-        _Float16* sh_act = reinterpret_cast<_Float16*>(base + L.off_sh_act);
-        float* sh_d = reinterpret_cast<float*>(base + L.off_sh_d);
-        auto H = [](const void* p) { return static_cast<const _Float16*>(p); };
-        auto U16 = [](const void* p) { return static_cast<const uint16_t*>(p); };
-        hipError_t e = hx::launch_input_had(xh, H(shared[0].suh), sh_a, nullptr, tokens, hidden_dim, st);
-        if (!e) e = hx::launch_linear_mfma(sh_a, nullptr, U16(shared[0].trellis), H(shared[0].svh), sh_g, tokens, hidden_dim,
-                                           intermediate_dim, shared_bits[0], cb, true, nullptr, nullptr, st);
-        if (!e) e = hx::launch_input_had(xh, H(shared[1].suh), sh_a, nullptr, tokens, hidden_dim, st);
-        if (!e) e = hx::launch_linear_mfma(sh_a, nullptr, U16(shared[1].trellis), H(shared[1].svh), sh_u, tokens, hidden_dim,
-                                           intermediate_dim, shared_bits[1], cb, true, nullptr, nullptr, st);
-        if (!e) e = hx::launch_swiglu_clamp(sh_g, sh_u, sh_act, (size_t)tokens * intermediate_dim, act_limit, st);
-        if (!e) e = hx::launch_input_had(sh_act, H(shared[2].suh), sh_a, nullptr, tokens, intermediate_dim, st);
-        if (!e) e = hx::launch_linear_mfma(sh_a, nullptr, U16(shared[2].trellis), H(shared[2].svh), sh_d, tokens,
-                                           intermediate_dim, hidden_dim, shared_bits[2], cb, true, nullptr, nullptr, st);
-        if ((r = hip_status(e, "hx_moe_layer(shared expert)"))) return r;
-        shared_rows = sh_d;
-    }
     hx::PrefillArgs p{};
     p.x = xh;
     p.T = tokens;
@@ -745,10 +722,18 @@ int hx_moe_layer(void* y, float* y_routed, const void* x, const void* scores, co
     fill_tables(tables, p.tr, p.suh, p.svh, p.bits_tab, p.bits_uniform, K_gate, K_up, K_down);
     p.act_limit = act_limit;
     p.cb = cb;
+    p.shared = shared != nullptr;
+    if (shared)
+        for (int i = 0; i < 3; ++i) {
+            p.sh_tr[i] = shared[i].trellis;
+            p.sh_suh[i] = static_cast<const _Float16*>(shared[i].suh);
+            p.sh_svh[i] = static_cast<const _Float16*>(shared[i].svh);
+            p.sh_bits[i] = shared_bits[i];
+        }
     p.ws = base;
     p.lay = &L;
     Phase ph(7, st);
-    return hip_status(hx::run_moe_prefill(p, nullptr, shared_rows, static_cast<_Float16*>(y), y_routed, false, st),
+    return hip_status(hx::run_moe_prefill(p, nullptr, static_cast<_Float16*>(y), y_routed, false, st),
                       "hx_moe_layer(prefill)");
 }
 

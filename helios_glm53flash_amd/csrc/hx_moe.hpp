@@ -19,7 +19,7 @@ struct MoeWs {
     // prefill path
     int max_jobs = 0;
     size_t off_perm = 0, off_jobs = 0, off_njobs = 0, off_row_expert = 0, off_xg = 0, off_xu = 0, off_G = 0,
-           off_A = 0, off_rs = 0, off_D = 0, off_sh_a = 0, off_sh_g = 0, off_sh_u = 0, off_sh_act = 0, off_sh_d = 0;
+           off_A = 0, off_rs = 0, off_D = 0, off_sh_g = 0, off_sh_d = 0;
     size_t prefill_end = 0;
     size_t total = 0;
 
@@ -44,6 +44,12 @@ struct PrefillArgs {
     float act_limit;
     int act_fn;        // HX_ACT_* of the routed experts
     int cb;
+    // shared expert (gate, up, down), run on every token when `shared`
+    bool shared;
+    const void* sh_tr[3];
+    const _Float16* sh_suh[3];
+    const _Float16* sh_svh[3];
+    int sh_bits[3];
     char* ws;
     const MoeWs* lay;
 };
@@ -57,9 +63,9 @@ int resident_blocks(const void* kernel, int threads, size_t lds);
 int decode_resident(const void* kernel, int threads, size_t lds, int max_per_cu);
 size_t decode_lds_pad(const void* kernel, size_t lds, int max_per_cu);
 // Routed experts for T > 8 tokens: writes per-row fp32 contributions (sorted order) when contrib is
-// non-null, y = fp16(routed + shared_rows) when y is non-null, and the fp32 routed sum into
+// non-null, y = fp16(routed + shared expert) when y is non-null, and the fp32 routed sum into
 // y_routed (added to its contents when accumulate) when y_routed is non-null.
-hipError_t run_moe_prefill(const PrefillArgs& p, float* contrib, const float* shared_rows, _Float16* y,
-                           float* y_routed, bool accumulate, hipStream_t st);
+hipError_t run_moe_prefill(const PrefillArgs& p, float* contrib, _Float16* y, float* y_routed, bool accumulate,
+                           hipStream_t st);
 
 }  // namespace hx

@@ -9,10 +9,12 @@
 //              workgroup act[r] = fp16(H((act(g) * u) . suh_d)), g = fp16(H(G)) . svh_g ... (fp16
 //              chain, transforms on the matrix cores), and the row sums of act
 //   gemm d     D = act . W_d[e]                    (fp16 output)
+//   The shared expert's rows (every token) follow the R sorted rows through gather, gate/up and down as jobs of
+//   their own, first in the grid, with fp32 between its GEMMs and transforms (as the reference's shared MLP).
 //   combine    y[t] = fp16(sum_j H(D[r_j]) * w_j / sqrt(128) . svh_d[e_j]  + shared[t])
 // Reference semantics: src/cuda/quant/exl3_moe_kernel.cuh:57-262, hadamard_inner.cuh:284-481,
 // src/engine/glue2.cu:297-306, runner.cpp:957-958.
-#include "hx_mfma.hpp"
+#include "hx_gemm_impl.hpp"
 #include "hx_kernels.hpp"
 #include "hx_moe.hpp"
 
@@ -20,28 +22,25 @@ namespace hx {
 
 static size_t al(size_t v) { return (v + 255) & ~(size_t)255; }
 
-struct Job {
+struct Job {  // expert -1: the shared expert, row0 >= R
     int expert, row0, rows, bm;  // bm: row tile (128, or 96 / 64 / 32 for a remainder of at most that many rows)
 };
 
 void MoeWs::prefill_layout(size_t o)
 {
-    max_jobs = (R + MF_BM - 1) / MF_BM + E;
-    const int kmax = hidden > inter ? hidden : inter;
+    max_jobs = (R + MF_BM - 1) / MF_BM + E + (T + MF_BM - 1) / MF_BM;
+    const size_t RT = (size_t)R + T;  // routed rows, then the shared expert's
     off_perm = o;       o = al(o + sizeof(int) * 2 * (size_t)((R + 1023) / 1024) * E);
     off_jobs = o;       o = al(o + sizeof(Job) * max_jobs);
     off_njobs = o;      o = al(o + sizeof(int));
     off_row_expert = o; o = al(o + sizeof(int) * R);
-    off_xg = o;         o = al(o + sizeof(_Float16) * (size_t)R * hidden);
-    off_xu = o;         o = al(o + sizeof(_Float16) * (size_t)R * hidden);
+    off_xg = o;         o = al(o + sizeof(_Float16) * RT * hidden);
+    off_xu = o;         o = al(o + sizeof(_Float16) * RT * hidden);
     off_G = o;          o = al(o + sizeof(_Float16) * (size_t)R * inter);
-    off_A = o;          o = al(o + sizeof(_Float16) * (size_t)R * inter);
-    off_rs = o;         o = al(o + sizeof(float) * (size_t)R * (2 * (hidden / 128) + inter / 128));
+    off_A = o;          o = al(o + sizeof(_Float16) * RT * inter);
+    off_rs = o;         o = al(o + sizeof(float) * RT * (2 * (hidden / 128) + inter / 128));
     off_D = off_xg;     // D reuses xg (xg is consumed by the gate GEMM before the down GEMM runs)
-    off_sh_a = o;       o = al(o + sizeof(_Float16) * (size_t)T * kmax);
     off_sh_g = o;       o = al(o + sizeof(float) * (size_t)T * inter);
-    off_sh_u = o;       o = al(o + sizeof(float) * (size_t)T * inter);
-    off_sh_act = o;     o = al(o + sizeof(_Float16) * (size_t)T * inter);
     off_sh_d = o;       o = al(o + sizeof(float) * (size_t)T * hidden);
     prefill_end = o;
 }
@@ -50,9 +49,11 @@ void MoeWs::prefill_layout(size_t o)
 
 // Every block scans the expert counts (E <= 512) in LDS; block 0 writes the tile jobs, and each
 // block maps its 256 rows to their expert.
-__global__ __launch_bounds__(512) void prefill_plan_kernel(const int64_t* expert_count, int E, int R, Job* jobs,
-                                                          int* njobs, int* row_expert)
+__global__ __launch_bounds__(512) void prefill_plan_kernel(const int64_t* expert_count, int E, int R, int shared_rows,
+                                                          Job* jobs, int* njobs, int* row_expert)
 {
+    auto tile = [](int rows) { return rows <= 32 ? 32 : rows <= 64 ? 64 : rows <= 96 ? 96 : MF_BM; };
+    const int nsh = (shared_rows + MF_BM - 1) / MF_BM;  // the shared expert's jobs come first
     __shared__ int off[513];   // exclusive scan of the row counts
     __shared__ int joff[513];  // exclusive scan of the job counts
     const int t = threadIdx.x;
@@ -72,9 +73,13 @@ __global__ __launch_bounds__(512) void prefill_plan_kernel(const int64_t* expert
     if (blockIdx.x == 0) {
         for (int k = 0; k < nj; ++k) {
             const int rows = min(MF_BM, c - k * MF_BM);
-            jobs[j0 + k] = Job{t, r0 + k * MF_BM, rows, rows <= 32 ? 32 : rows <= 64 ? 64 : rows <= 96 ? 96 : MF_BM};
+            jobs[nsh + j0 + k] = Job{t, r0 + k * MF_BM, rows, tile(rows)};
         }
-        if (t == 511) *njobs = joff[511];
+        for (int k = t; k < nsh; k += 512) {
+            const int rows = min(MF_BM, shared_rows - k * MF_BM);
+            jobs[k] = Job{-1, R + k * MF_BM, rows, tile(rows)};
+        }
+        if (t == 511) *njobs = nsh + joff[511];
     }
     __syncthreads();
     off[t] = r0;
@@ -104,20 +109,29 @@ __global__ __launch_bounds__(512) void prefill_plan_kernel(const int64_t* expert
 __global__ __launch_bounds__(256, 4) void prefill_gather_kernel(const _Float16* x, const int64_t* token_sorted,
                                                             const int* row_expert, const void* const* suh_g,
                                                             const void* const* suh_u, _Float16* xg, _Float16* xu,
-                                                            int hidden, bool gated, float* rs_g, float* rs_u, long R)
+                                                            int hidden, bool gated, float* rs_g, float* rs_u, long R,
+                                                            long RT, const _Float16* sh_suh_g, const _Float16* sh_suh_u)
 {
     const int lane = threadIdx.x & 63;
     const int nblk = hidden >> 7;
     const long unit = (long)blockIdx.x * 4 + (threadIdx.x >> 6);  // (row block, column block)
     const long rb = unit / nblk;
     const int kb = (int)(unit % nblk);
-    if (rb * 16 >= R) return;
+    if (rb * 16 >= RT) return;
     const int c = lane & 15, g = lane >> 4;
-    const long r = min(rb * 16 + c, R - 1);  // A row of this lane (rows past R repeat the last, not stored)
-    const int e = row_expert[r];
-    const _Float16* xr = x + (size_t)token_sorted[r] * hidden + kb * 128 + 8 * g;
-    const _Float16* sg = static_cast<const _Float16*>(gated ? suh_g[e] : suh_u[e]) + kb * 128 + 8 * g;
-    const _Float16* su = static_cast<const _Float16*>(suh_u[e]) + kb * 128 + 8 * g;
+    // A row of this lane (rows past the end repeat the last, not stored); rows from R on are the shared expert's
+    const long r = min(rb * 16 + c, RT - 1);
+    long token = r - R;
+    const _Float16 *sg = sh_suh_g, *su = sh_suh_u;
+    if (r < R) {
+        const int e = row_expert[r];
+        token = token_sorted[r];
+        sg = static_cast<const _Float16*>(gated ? suh_g[e] : suh_u[e]);
+        su = static_cast<const _Float16*>(suh_u[e]);
+    }
+    const _Float16* xr = x + (size_t)token * hidden + kb * 128 + 8 * g;
+    sg += kb * 128 + 8 * g;
+    su += kb * 128 + 8 * g;
     hx_h8 xv[4];
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) xv[kk] = *reinterpret_cast<const hx_h8*>(xr + 32 * kk);
@@ -175,7 +189,7 @@ __global__ __launch_bounds__(256, 4) void prefill_gather_kernel(const _Float16* 
     for (int q = 0; q < 4; ++q) {
         const int row16 = 4 * q + (lane >> 4), c8 = 8 * (lane & 15);
         const long row = rb * 16 + row16;
-        if (row < R) {
+        if (row < RT) {
             const size_t o = (size_t)row * hidden + kb * 128 + c8;
             if (gated) *reinterpret_cast<hx_u4v*>(xg + o) = *reinterpret_cast<const hx_u4v*>(&sw[0][row16][c8]);
             *reinterpret_cast<hx_u4v*>(xu + o) = *reinterpret_cast<const hx_u4v*>(&sw[1][row16][c8]);
@@ -194,7 +208,7 @@ __global__ __launch_bounds__(256, 4) void prefill_gather_kernel(const _Float16* 
         for (int i = 0; i < 4; ++i)
             if (c == i) vg_ = sum_g[i], vu_ = sum_u[i];
         const long row = rb * 16 + 4 * g + c;
-        if (row < R) {
+        if (row < RT) {
             if (gated) rs_g[(size_t)row * nblk + kb] = vg_;
             rs_u[(size_t)row * nblk + kb] = vu_;
         }
@@ -206,25 +220,40 @@ __global__ __launch_bounds__(256, 4) void prefill_gather_kernel(const _Float16* 
 struct GroupedGemmArgs {
     const Job* jobs;
     const int* njobs;
-    const _Float16* A[2];
-    _Float16* out[2];
-    const void* const* tr[2];
-    const int32_t* bits_tab[2];
-    int bits_uniform[2];
-    int K, N, nproj;
-    const float* rs[2];  // precomputed row sums of A: rs_n partial sums per row
+    const _Float16* A;
+    _Float16* out;
+    const void* const* tr;
+    const int32_t* bits_tab;
+    int bits_uniform;
+    int K, N;
+    const float* rs;  // precomputed row sums of A: rs_n partial sums per row
     int rs_n;
+    // the shared expert (jobs with expert -1, rows from R on): fp32 rows svh . H(D) of every token
+    const void* sh_tr;
+    const _Float16* sh_svh;
+    int sh_bits, R;
+    float* sh_out;
 };
 
 template <int BITS, int CB, int BM>
-__device__ __forceinline__ void grouped_tile(const GroupedGemmArgs& g, const Job& job, int proj, int cg, MfmaSmemQ& sm)
+__device__ __forceinline__ void grouped_tile(const GroupedGemmArgs& g, const Job& job, int cg, MfmaSmemQ& sm)
 {
-    const _Float16* A = g.A[proj] + (size_t)job.row0 * g.K;
-    const uint32_t* tr = static_cast<const uint32_t*>(g.tr[proj][job.expert]);
+    const _Float16* A = g.A + (size_t)job.row0 * g.K;
+    const bool shared = job.expert < 0;
+    const uint32_t* tr = static_cast<const uint32_t*>(shared ? g.sh_tr : g.tr[job.expert]);
     hx_f4 acc[BM / 16][2];
     mfma_tile_q<BITS, CB, BM, true, BM <= 32 ? 4 : QT_PF>(A, g.K, job.rows, tr, g.K, g.N, cg * 8, sm, acc,
-                                            g.rs[proj] + (size_t)job.row0 * g.rs_n, g.rs_n);
-    _Float16* out = g.out[proj] + (size_t)job.row0 * g.N + cg * 128;
+                                            g.rs + (size_t)job.row0 * g.rs_n, g.rs_n);
+    if (shared) {
+        MfmaGemmArgs o{};
+        o.svh = g.sh_svh;
+        o.y = g.sh_out;
+        o.N = g.N;
+        o.y_fp32 = true;
+        linear_tile_store<CB, BM>(acc, sm, o, job.row0 - g.R, job.rows, cg);
+        return;
+    }
+    _Float16* out = g.out + (size_t)job.row0 * g.N + cg * 128;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int half = 0; half < (BM + 63) / 64; ++half) {
         qt_stage_c_half<BM>(acc, half, sm);
@@ -250,19 +279,16 @@ template <int CB>
 __global__ __launch_bounds__(MF_THREADS, qt_occ<CB>()) void grouped_gemm_kernel(GroupedGemmArgs g)
 {
     __shared__ MfmaSmemQ sm;
-    int bx, job_i;
-    if (!grouped_tile_index(*g.njobs, bx, job_i)) return;
+    int cg, job_i;
+    if (!grouped_tile_index(*g.njobs, cg, job_i)) return;
     const Job job = g.jobs[job_i];
-    const int ntiles = g.N / 128;
-    const int proj = bx / ntiles;
-    const int cg = bx % ntiles;
-    const int bits = g.bits_tab[proj] ? g.bits_tab[proj][job.expert] : g.bits_uniform[proj];
+    const int bits = job.expert < 0 ? g.sh_bits : g.bits_tab ? g.bits_tab[job.expert] : g.bits_uniform;
 #define HX_GG_CASE(B)                                                                      \
     case B:                                                                                \
-        if (job.bm == 32) grouped_tile<B, CB, 32>(g, job, proj, cg, sm);                    \
-        else if (job.bm == 64) grouped_tile<B, CB, 64>(g, job, proj, cg, sm);               \
-        else if (job.bm == 96) grouped_tile<B, CB, 96>(g, job, proj, cg, sm);               \
-        else grouped_tile<B, CB, MF_BM>(g, job, proj, cg, sm);                              \
+        if (job.bm == 32) grouped_tile<B, CB, 32>(g, job, cg, sm);                    \
+        else if (job.bm == 64) grouped_tile<B, CB, 64>(g, job, cg, sm);               \
+        else if (job.bm == 96) grouped_tile<B, CB, 96>(g, job, cg, sm);               \
+        else grouped_tile<B, CB, MF_BM>(g, job, cg, sm);                              \
         break;
     switch (bits) {
         HX_GG_CASE(1) HX_GG_CASE(2) HX_GG_CASE(3) HX_GG_CASE(4)
@@ -292,6 +318,12 @@ struct GuArgs {
     const float* rs_g;   // [R][K / 128] row sums of xg, xu per 128-column block
     const float* rs_u;
     float* rs_act;       // [R][inter / 128] row sums of act per 128-column block
+    // the shared expert (jobs with expert -1, rows from R on)
+    const void* sh_tr[2];
+    const _Float16* sh_svh[2];
+    const _Float16* sh_suh_d;
+    int sh_bits[2], R;
+    float* sh_g;         // [T][inter] fp32 g of the tiles in flight
 };
 
 // accumulator of the gate/up tiles (quarter-operand layout); LDS: the tile's A buffers, reused as the
@@ -302,6 +334,7 @@ struct GuSmem {
     union {
         _Float16 ab[QT_NB][MF_BM * MF_LDA];
         _Float16 hx[128 * MF_LDA2];
+        float c[64 * MF_LDC];
     };
     float rowsum[MF_BM];
 };
@@ -328,6 +361,91 @@ __device__ __forceinline__ void gu_tile_bits(int bits, const _Float16* A, int K,
         case 7: gu_tile<7, CB, BM>(A, K, rows, tr, N, cg, sm, acc, rs); break;
         default: gu_tile<8, CB, BM>(A, K, rows, tr, N, cg, sm, acc, rs); break;
     }
+}
+
+// The shared expert's epilogues, in fp32 until the activation as the reference's shared MLP (two GEMMs with
+// fp32 outputs, swiglu_clamp, input transform of the down GEMM; runner.cpp:723-738): 4 lanes per row
+// (had128_quad), 64 rows at a time.  The gate's g = svh . H(G) waits in fp32 scratch while the up tile runs
+// (each lane reads back what it stored).  UP: act = fp16(silu(min(g, L)) * clamp(u)), then fp16(H(act . suh_d)).
+template <int CB, int BM, bool UP>
+__device__ __forceinline__ void gu_shared(const GuArgs& a, const Job& job, int cg, GuSmem& sm,
+                                          const hx_f4 (&acc)[BM / 16][2])
+{
+    const int r = threadIdx.x >> 2, p = threadIdx.x & 3, c = cg * 128 + 8 * p;
+    const _Float16* svh = a.sh_svh[UP] + c;
+#pragma unroll
+    for (int half = 0; half < (BM + 63) / 64; ++half) {
+        if (half) __syncthreads();
+        qt_stage_c_half<BM>(acc, half, sm);
+        __syncthreads();
+        const int row = 64 * half + r;
+        const bool live = row < job.rows;
+        float v[32];
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const hx_f4 q = *reinterpret_cast<const hx_f4*>(&sm.c[r * MF_LDC + 32 * m + 8 * p + 4 * e]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[8 * m + 4 * e + i] = q[i];
+            }
+        if constexpr (CB == 2) {
+            const float b = CB2_BIAS * sm.rowsum[min(row, MF_BM - 1)];
+#pragma unroll
+            for (int j = 0; j < 32; ++j) v[j] = fmaf(v[j], CB2_SCALE, b);
+        }
+        had128_quad(v);
+        float* gs = a.sh_g + (size_t)(job.row0 - a.R + (live ? row : 0)) * a.N + c;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const hx_h8 sv = *reinterpret_cast<const hx_h8u*>(svh + 32 * m);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[8 * m + i] *= (float)sv[i];
+        }
+        if constexpr (!UP) {
+            if (live) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        *reinterpret_cast<hx_f4*>(gs + 32 * m + 4 * e) =
+                            hx_f4{v[8 * m + 4 * e], v[8 * m + 4 * e + 1], v[8 * m + 4 * e + 2], v[8 * m + 4 * e + 3]};
+            }
+        } else {
+            const float L = a.act_limit;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                const hx_h8 sd = *reinterpret_cast<const hx_h8u*>(a.sh_suh_d + c + 32 * m);
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const hx_f4 g4 = *reinterpret_cast<const hx_f4*>(gs + 32 * m + 4 * e);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float g = fminf(g4[i], L), u = fminf(fmaxf(v[8 * m + 4 * e + i], -L), L);
+                        const _Float16 act = (_Float16)(g / (1.0f + __expf(-g)) * u);
+                        v[8 * m + 4 * e + i] = (float)(_Float16)(act * sd[4 * e + i]);
+                    }
+                }
+            }
+            had128_quad(v);
+            float sum = 0.0f;
+            _Float16* out = a.act + (size_t)(job.row0 + (live ? row : 0)) * a.N + c;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                hx_h8 h;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    h[i] = (_Float16)v[8 * m + i];
+                    sum += (float)h[i];
+                }
+                if (live) *reinterpret_cast<hx_h8*>(out + 32 * m) = h;
+            }
+            sum += __shfl_xor(sum, 1, 64);
+            sum += __shfl_xor(sum, 2, 64);
+            if (live && p == 0) a.rs_act[(size_t)(job.row0 + row) * (a.N >> 7) + cg] = sum;
+        }
+    }
+    __syncthreads();  // sm.c is read before the next tile's buffers overwrite it
 }
 
 // Gate and up tiles of one (job, 128-column block), then the SiLU-gate and the down-projection input
@@ -443,6 +561,20 @@ __device__ __forceinline__ void gu_fused(const GuArgs& a, const Job& job, int cg
     }
 }
 
+// A job of the shared expert (code of its own: folded into gu_fused its pointers spilled registers inside the
+// routed tiles' chunk loops, 3.07 -> 3.34 ms at 4096 tokens).
+template <int CB, int BM>
+__device__ __forceinline__ void gu_shared_job(const GuArgs& a, const Job& job, int cg, GuSmem& sm)
+{
+    GuAcc<BM> acc;
+    gu_tile_bits<CB, BM>(a.sh_bits[0], a.xg + (size_t)job.row0 * a.K, a.K, job.rows, a.sh_tr[0], a.N, cg, sm, acc,
+                         a.rs_g + (size_t)job.row0 * (a.K / 128));
+    gu_shared<CB, BM, false>(a, job, cg, sm, acc);
+    gu_tile_bits<CB, BM>(a.sh_bits[1], a.xu + (size_t)job.row0 * a.K, a.K, job.rows, a.sh_tr[1], a.N, cg, sm, acc,
+                         a.rs_u + (size_t)job.row0 * (a.K / 128));
+    gu_shared<CB, BM, true>(a, job, cg, sm, acc);
+}
+
 template <int CB>
 __global__ __launch_bounds__(MF_THREADS, qt_occ<CB>()) void grouped_gu_kernel(GuArgs a)
 {
@@ -450,6 +582,12 @@ __global__ __launch_bounds__(MF_THREADS, qt_occ<CB>()) void grouped_gu_kernel(Gu
     int cg, job_i;
     if (!grouped_tile_index(*a.njobs, cg, job_i)) return;
     const Job job = a.jobs[job_i];
+    if (job.expert < 0) {
+        if (job.bm == 32) gu_shared_job<CB, 32>(a, job, cg, sm);
+        else if (job.bm == 64) gu_shared_job<CB, 64>(a, job, cg, sm);
+        else gu_shared_job<CB, MF_BM>(a, job, cg, sm);
+        return;
+    }
     if (job.bm == 32) gu_fused<CB, 32>(a, job, cg, sm);
     else if (job.bm == 64) gu_fused<CB, 64>(a, job, cg, sm);
     else if (job.bm == 96) gu_fused<CB, 96>(a, job, cg, sm);
@@ -685,8 +823,8 @@ __global__ __launch_bounds__(256) void prefill_contrib_kernel(const _Float16* D,
 
 // ------------------------------------------------------------------ driver
 
-hipError_t run_moe_prefill(const PrefillArgs& p, float* contrib, const float* shared_rows, _Float16* y,
-                           float* y_routed, bool accumulate, hipStream_t st)
+hipError_t run_moe_prefill(const PrefillArgs& p, float* contrib, _Float16* y, float* y_routed, bool accumulate,
+                           hipStream_t st)
 {
     const MoeWs& L = *p.lay;
     char* ws = p.ws;
@@ -699,16 +837,20 @@ hipError_t run_moe_prefill(const PrefillArgs& p, float* contrib, const float* sh
     _Float16* A = reinterpret_cast<_Float16*>(ws + L.off_A);
     _Float16* D = reinterpret_cast<_Float16*>(ws + L.off_D);
     float* rs_g = reinterpret_cast<float*>(ws + L.off_rs);
-    float* rs_u = rs_g + (size_t)p.R * (p.hidden / 128);
-    float* rs_act = rs_u + (size_t)p.R * (p.hidden / 128);
+    const long RT = (long)p.R + (p.shared ? p.T : 0);  // routed rows, then the shared expert's
+    float* rs_u = rs_g + (size_t)RT * (p.hidden / 128);
+    float* rs_act = rs_u + (size_t)RT * (p.hidden / 128);
+    float* sh_d = reinterpret_cast<float*>(ws + L.off_sh_d);
+    const float* shared_rows = p.shared ? sh_d : nullptr;
     if (p.E > 512) return hipErrorInvalidValue;
 
     hipLaunchKernelGGL(prefill_plan_kernel, dim3((unsigned)((p.R + 511) / 512)), dim3(512), 0, st, p.expert_count,
-                       p.E, p.R, jobs, njobs, row_expert);
+                       p.E, p.R, p.shared ? p.T : 0, jobs, njobs, row_expert);
     if (p.R > 0)
-        hipLaunchKernelGGL(prefill_gather_kernel, dim3((unsigned)((((long)p.R + 15) / 16 * (p.hidden / 128) + 3) / 4)),
+        hipLaunchKernelGGL(prefill_gather_kernel, dim3((unsigned)(((RT + 15) / 16 * (p.hidden / 128) + 3) / 4)),
                            dim3(256), 0, st, p.x, p.token_sorted,
-                           row_expert, p.suh[0], p.suh[1], xg, xu, p.hidden, p.act_fn != HX_ACT_RELU2_NOGATE, rs_g, rs_u, (long)p.R);
+                           row_expert, p.suh[0], p.suh[1], xg, xu, p.hidden, p.act_fn != HX_ACT_RELU2_NOGATE, rs_g, rs_u, (long)p.R,
+                           RT, p.sh_suh[0], p.sh_suh[1]);
 
     GuArgs gu{};
     gu.jobs = jobs;
@@ -733,6 +875,14 @@ hipError_t run_moe_prefill(const PrefillArgs& p, float* contrib, const float* sh
     gu.rs_g = rs_g;
     gu.rs_u = rs_u;
     gu.rs_act = rs_act;
+    for (int i = 0; i < 2; ++i) {
+        gu.sh_tr[i] = p.sh_tr[i];
+        gu.sh_svh[i] = p.sh_svh[i];
+        gu.sh_bits[i] = p.sh_bits[i];
+    }
+    gu.sh_suh_d = p.sh_suh[2];
+    gu.R = p.R;
+    gu.sh_g = reinterpret_cast<float*>(ws + L.off_sh_g);
     dim3 grid_gu(p.inter / 128, L.max_jobs);
     if (p.cb == 1) hipLaunchKernelGGL(grouped_gu_kernel<1>, grid_gu, dim3(MF_THREADS), 0, st, gu);
     else hipLaunchKernelGGL(grouped_gu_kernel<2>, grid_gu, dim3(MF_THREADS), 0, st, gu);
@@ -740,16 +890,20 @@ hipError_t run_moe_prefill(const PrefillArgs& p, float* contrib, const float* sh
     GroupedGemmArgs d{};
     d.jobs = jobs;
     d.njobs = njobs;
-    d.A[0] = A;
-    d.out[0] = D;
-    d.tr[0] = p.tr[2];
-    d.bits_tab[0] = p.bits_tab[2];
-    d.bits_uniform[0] = p.bits_uniform[2];
+    d.A = A;
+    d.out = D;
+    d.tr = p.tr[2];
+    d.bits_tab = p.bits_tab[2];
+    d.bits_uniform = p.bits_uniform[2];
     d.K = p.inter;
     d.N = p.hidden;
-    d.nproj = 1;
-    d.rs[0] = rs_act;
+    d.rs = rs_act;
     d.rs_n = p.inter / 128;
+    d.sh_tr = p.sh_tr[2];
+    d.sh_svh = p.sh_svh[2];
+    d.sh_bits = p.sh_bits[2];
+    d.R = p.R;
+    d.sh_out = sh_d;
     dim3 grid_d(p.hidden / 128, L.max_jobs);
     if (p.cb == 1) hipLaunchKernelGGL(grouped_gemm_kernel<1>, grid_d, dim3(MF_THREADS), 0, st, d);
     else hipLaunchKernelGGL(grouped_gemm_kernel<2>, grid_d, dim3(MF_THREADS), 0, st, d);

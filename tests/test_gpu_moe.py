@@ -362,3 +362,12 @@ def test_moe_grouped_every_bit_width(hx, cb, T):
     got = y.cpu().numpy()
     assert np.isfinite(got).all()
     assert_close(got, ref, what=f"every width, cb={cb}, T={T}")
+
+
+@pytest.mark.parametrize("T,topk,shared_bits", [(9, 3, (2, 2, 2)), (33, 2, (4, 1, 8)), (70, 4, (3, 5, 2)),
+                                                (129, 1, (6, 7, 3)), (225, 2, (2, 3, 2))])
+@pytest.mark.parametrize("inter", [128, 384])
+def test_prefill_shared_expert_rows(hx, T, topk, shared_bits, inter):
+    """The shared expert's rows behind the routed ones: row counts that straddle 16-row groups, every height of
+    its last row tile, widths of its own per projection."""
+    _run_layer(hx, 12, 256, inter, topk, T, 2, shared_bits, seed=T + inter)
