@@ -666,9 +666,35 @@ int hx_moe_layer(void* y, float* y_routed, const void* x, const void* scores, co
     if (L.few_tokens()) {
         hx::MoeDecodeArgs a = L.decode_args(base);
         a.x = xh;
-        a.scores = static_cast<const _Float16*>(scores);
-        a.bias = static_cast<const _Float16*>(bias);
-        a.routed_scale = routed_scale;
+        if (tokens <= 4) {
+            a.scores = static_cast<const _Float16*>(scores);
+            a.bias = static_cast<const _Float16*>(bias);
+            a.routed_scale = routed_scale;
+            a.out_idx = idx;
+            a.out_w = wt;
+        } else {
+            // Routed and sorted once ahead of the layer kernel: its 2000-4000 workgroups would each select for 5-8
+            // tokens and rank up to 64 routes (8 tokens 272 -> 214 us; at 2-4 tokens the two launches cost more
+            // than they save, 102 -> 111 us).
+            {
+                Phase ph(0, st);
+                r = hip_status(hx::launch_routing(static_cast<const _Float16*>(scores),
+                                                  static_cast<const _Float16*>(bias), idx, wt, tokens, num_experts,
+                                                  topk, routed_scale, st),
+                               "hx_moe_layer(routing)");
+            }
+            if (r) return r;
+            {
+                Phase ph(1, st);
+                r = hip_status(hx::launch_permute(idx, wt, tokens, topk, num_experts, cnt, ts, wsorted, r2s, nullptr, st),
+                               "hx_moe_layer(permute)");
+            }
+            if (r) return r;
+            a.expert_count = cnt;
+            a.token_sorted = ts;
+            a.weight_sorted = wsorted;
+            a.route_to_sorted = r2s;
+        }
         fill_tables(tables, a.tr, a.suh, a.svh, a.bits_tab, a.bits_uniform, K_gate, K_up, K_down);
         uint32_t mgu = phase_mask(tables, K_gate, K_up), md = phase_mask(tables, K_down, 0);
         if (shared) {
@@ -682,8 +708,6 @@ int hx_moe_layer(void* y, float* y_routed, const void* x, const void* scores, co
             md |= 1u << shared_bits[2];
         }
         a.act_limit = act_limit;
-        a.out_idx = idx;
-        a.out_w = wt;
         a.combine = true;
         a.y = static_cast<_Float16*>(y);
         a.y_routed = y_routed;

@@ -174,6 +174,12 @@ size_t decode_lds_pad(const void* kernel, size_t lds, int max_per_cu)
 // (With the earlier ring, whose waits drained every load in flight once per group, 864 + 864 was
 // the faster one.)
 // A fused variant (workgroup w runs gate/up unit w then down unit w, reusing its plan) took 60 us.
+// Several tokens: every column group gets the same number of units, the whole number nearest to a round of
+// residents but at most 2 (each unit routes or reads the plan, transforms its rows and publishes), or as many as
+// keep a unit's input rows within 32 KB of LDS.  288 experts + shared, 2-bit, 4096 x 2048: 2 tokens 66.0 us with
+// 2 per group, 72.6 with 1; 3 tokens 83.7 with 1 (85.5 with 1024 units over its 800 groups); 4 tokens 102 with
+// 1 (2, 3 and 4 were slower already); 8 tokens 214 with 2, 243 with 4.  64 experts, 2048 x 1024, 2 tokens: 34.0
+// with 2, 37.7 with 3, 45.5 with 4.
 // Returns the longest unit's k extent.
 int decode_units(MoeDecodeArgs& a, int resident)
 {
@@ -181,7 +187,18 @@ int decode_units(MoeDecodeArgs& a, int resident)
     const long cg_gu = slots * 2 * (a.inter / 128), kb_gu = a.hidden / 128;
     const long cg_d = slots * (a.hidden / 128), kb_d = a.inter / 128;
     auto clampu = [](long u, long c, long kb) { return u < c ? c : (u > c * kb ? c * kb : u); };
-    long ug = clampu(resident, cg_gu, kb_gu), ud = clampu(resident - resident / 16, cg_d, kb_d);
+    long ug = resident, ud = resident - resident / 16;
+    if (a.T > 1) {
+        const long mt = a.T <= 4 ? 4 : 8;
+        auto per_group = [&](long cg, long kb) {
+            const long fit = (kb * 128 * mt * 2 + 32767) / 32768, near = (2 * resident + cg) / (2 * cg), round = near < 2 ? near : 2;
+            return fit > round ? fit : round;
+        };
+        ug = cg_gu * per_group(cg_gu, kb_gu);
+        ud = cg_d * per_group(cg_d, kb_d);
+    }
+    ug = clampu(ug, cg_gu, kb_gu);
+    ud = clampu(ud, cg_d, kb_d);
     a.units_gu = (int)ug;
     a.units_d = (int)ud;
     const long bg = (kb_gu + ug / cg_gu - 1) / (ug / cg_gu), bd = (kb_d + ud / cg_d - 1) / (ud / cg_d);

@@ -32,6 +32,12 @@ constexpr int DEC_STATUS_BAD_BITS = 2; // a per-expert bit table held a width ou
 // suh of the projection it streams, and the scale rows of its epilogue (gate/up units: svh of gate,
 // svh of up, suh of down; down units: svh of down).
 constexpr int DEC_TABS = 5;
+// Expert table entries parked in LDS while the plan is built (for up to this many experts): they use the input
+// rows' dynamic LDS, which is written only after the barrier that follows the plan.  An array of their own
+// (12.8 KB) held the 4-row kernel at 3 workgroups per CU instead of 4 and the 8-row kernel at 2: the layer at
+// 4 tokens 110 -> 102 us, at 8 tokens 464 -> 272 us.
+constexpr int DEC_TAB_MAX_E = 320;
+constexpr size_t DEC_TAB_LDS = DEC_TABS * DEC_TAB_MAX_E * sizeof(uint64_t);
 struct SlotTables {
     const void* tr;
     const void* suh;
@@ -312,12 +318,13 @@ HX_INLINE void load_slot_tables(const MoeDecodeArgs& a, SlotTables& t, int e, in
 // my_slot == DEC_SHARED, none for -1.  Layer mode routes the tokens; grouped mode reads the caller's
 // expert_count / token_sorted / weight_sorted.
 template <int MT>
-__device__ __forceinline__ void build_plan(const MoeDecodeArgs& a, DecodePlan& p, int my_slot, int proj)
+__device__ __forceinline__ void build_plan(const MoeDecodeArgs& a, DecodePlan& p, int my_slot, int proj,
+                                           uint32_t* a_lds)
 {
     __shared__ int sel_e[DEC_MAX_R];
     __shared__ float sel_w[DEC_MAX_R];
-    constexpr int TAB_MAX_E = 320, TPL = TAB_MAX_E / 64;
-    __shared__ uint64_t tab_lds[DEC_TABS][TAB_MAX_E];  // table entries of every expert
+    constexpr int TAB_MAX_E = DEC_TAB_MAX_E, TPL = TAB_MAX_E / 64;
+    uint64_t (*tab_lds)[TAB_MAX_E] = reinterpret_cast<uint64_t (*)[TAB_MAX_E]>(a_lds);  // table entries of every expert
     const int wave = hx_vwave(), lane = threadIdx.x & 63;
     const int R = a.T * a.topk;
     if (a.scores) {
@@ -972,7 +979,7 @@ __device__ __forceinline__ void moe_decode_body(const MoeDecodeArgs& a)
         // plan published by one workgroup would be read by all with device-coherent loads of the
         // same few lines (measured: 54 -> 97 us for the config-3 layer, the weight streams through
         // those lines' memory channel stall)
-        build_plan<MT>(a, plan, shared_unit ? DEC_SHARED : (has_shared ? us - 1 : us), proj);
+        build_plan<MT>(a, plan, shared_unit ? DEC_SHARED : (has_shared ? us - 1 : us), proj, a_lds);
     }
     if (blockIdx.x == 0 && a.out_idx) {
         const int R = a.T * a.topk;

@@ -21,7 +21,7 @@ static hipError_t launch_k(Kernel kernel, const MoeDecodeArgs& a0, hipStream_t s
         if (need == lds) break;
         lds = need;
     }
-    lds = decode_lds_pad(k, lds, 4);
+    lds = decode_lds_pad(k, lds > DEC_TAB_LDS ? lds : DEC_TAB_LDS, 4);
     hipLaunchKernelGGL(kernel, dim3(a.units_gu + a.units_d), dim3(DEC_THREADS), lds, st, a);
     return hipGetLastError();
 }

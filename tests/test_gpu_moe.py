@@ -371,3 +371,14 @@ def test_prefill_shared_expert_rows(hx, T, topk, shared_bits, inter):
     """The shared expert's rows behind the routed ones: row counts that straddle 16-row groups, every height of
     its last row tile, widths of its own per projection."""
     _run_layer(hx, 12, 256, inter, topk, T, 2, shared_bits, seed=T + inter)
+
+
+@pytest.mark.parametrize("T,topk,E,hidden,inter,bias", [(2, 8, 24, 256, 128, False), (3, 5, 8, 384, 256, True),
+                                                        (4, 8, 330, 256, 128, False), (5, 1, 4, 128, 128, False),
+                                                        (5, 8, 288, 4096, 256, True), (6, 7, 9, 640, 384, False),
+                                                        (7, 3, 512, 256, 128, True), (8, 8, 64, 2176, 128, False)])
+def test_decode_several_tokens(hx, T, topk, E, hidden, inter, bias):
+    """Few-token layer with routing inside (up to 4 tokens) and ahead of the kernel (5 to 8): one and several units
+    per column group, more experts than the parked tables hold, repeated calls on one workspace."""
+    for seed in (31, 32):
+        _run_layer(hx, E, hidden, inter, topk, T, 2, (2, 3, 2), seed=seed + T + E, bias=bias)
