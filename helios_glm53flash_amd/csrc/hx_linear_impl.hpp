@@ -1,6 +1,6 @@
 #pragma once
 // hx_linear_impl.hpp -- EXL3 quantized linear y = svh . H_N(H_K(x . suh) . W_hat) on gfx950,
-// small-M path (M <= 8): fused trellis decode + GEMV + split-K + output Hadamard epilogue in one
+// small-M path (M <= 16): fused trellis decode + GEMV + split-K + output Hadamard epilogue in one
 // launch.  Reference semantics: src/cuda/quant/exl3_gemv_kernel.cuh:138-402 and
 // exl3_gemm_kernel.cuh:8-80 (input transform, GEMM, output transform + svh).
 #include "hx_gemv.hpp"

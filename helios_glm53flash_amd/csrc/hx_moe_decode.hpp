@@ -1,6 +1,7 @@
 // hx_moe_decode.hpp -- fused MoE layer for few tokens (T <= 8, T*topk <= 64) on gfx950 in ONE
 // launch, without host synchronisation.  Every workgroup computes the router top-k and the
-// token-by-expert permutation from the fp16 scores (a few hundred bytes), then runs one unit:
+// token-by-expert permutation from the fp16 scores (a few hundred bytes; the layer calls it with the
+// caller's or an already built permutation from 5 tokens on), then runs one unit:
 //
 //   gate/up unit  one k range of one expert's gate or up GEMV with the trellis decode fused; the
 //                 last-arriving unit of a (slot, column group) adds the partial sums, runs the
