@@ -120,11 +120,12 @@ def test_mfma_parity(hx, M, bits, cb):
 
 @pytest.mark.parametrize("M,K,N,bits,cb", [(17, 4096, 256, 4, 2), (32, 640, 128, 2, 2), (33, 1152, 384, 3, 0),
                                            (64, 4096, 128, 5, 1), (65, 2176, 256, 8, 2), (97, 4096, 128, 2, 2),
-                                           (129, 1024, 256, 6, 2), (224, 3968, 128, 1, 2), (300, 512, 128, 7, 0)])
+                                           (129, 1024, 256, 6, 2), (224, 3968, 128, 1, 2), (300, 512, 128, 7, 0),
+                                           (17, 128, 128, 4, 2), (40, 256, 128, 2, 1), (90, 128, 256, 3, 2)])
 @pytest.mark.parametrize("y_fp32", [False, True])
 def test_mfma_row_tiles_and_k_splits(hx, M, K, N, bits, cb, y_fp32):
-    """Row tiles of every height with full and partial rows; K split into unequal chunk counts, and too short
-    to split."""
+    """Row tiles of every height with full and partial rows; K split into unequal chunk counts, too short to
+    split, and shorter than the rings."""
     for _ in range(2):  # the second call finds the arrival counters as the first left them
         path, got, ref = _run_linear(hx, M, K, N, bits, cb, y_fp32, seed=M + K)
         assert path == hx.HX_GEMM_PATH_MFMA
