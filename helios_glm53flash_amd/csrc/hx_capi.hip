@@ -217,12 +217,13 @@ int hx_exl3_gemm(void* y, const void* x, const hx_group_words* w, int M, int N, 
             return fail(HX_ERR_WORKSPACE, "hx_exl3_gemm: a_had is null and the workspace cannot hold M*K fp16");
         ah = reinterpret_cast<_Float16*>(static_cast<char*>(workspace) + hx::HX_COUNTER_BYTES);
     }
-    // row sums of the transformed input and K-split partials go to what the workspace has beyond the
-    // counters and (a_had null) the transformed input; a smaller workspace does without them
+    // Row sums of the transformed input and K-split partials go to what the workspace has beyond the counters and
+    // the transformed input; a smaller workspace does without them.  A call with its own a_had does not touch the
+    // workspace: such calls need nothing of it, so they may overlap, or sit in a graph that outlives it.
     float* rs = nullptr;
     void* partial = nullptr;
-    size_t o = hx::HX_COUNTER_BYTES + (a_had ? 0 : align256((size_t)M * K * sizeof(_Float16)));
-    if (workspace && workspace_bytes >= o + hx::mfma_rs_bytes(M, K)) {
+    size_t o = hx::HX_COUNTER_BYTES + align256((size_t)M * K * sizeof(_Float16));
+    if (!a_had && workspace_bytes >= o + hx::mfma_rs_bytes(M, K)) {
         rs = reinterpret_cast<float*>(static_cast<char*>(workspace) + o);
         o += hx::mfma_rs_bytes(M, K);
         const size_t pb = hx::mfma_partial_bytes(M, K, N);

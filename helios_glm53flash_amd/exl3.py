@@ -127,10 +127,8 @@ def gemm(y: torch.Tensor, x: torch.Tensor, w: GroupWords, M: int, N: int, K: int
     if a_had is not None:
         _need(a_had, "a_had", (torch.float16,))
     st = _stream(stream)
-    if M <= GEMV_MAX_M or a_had is None or not torch.cuda.is_current_stream_capturing():
-        ws = workspace(_gemm_workspace_bytes(M, N, K), x.device, st)
-    else:  # not needed then, only faster: take what the stream has, allocate nothing under capture
-        ws = _workspaces.get((x.device.index, st))
+    # with a_had an MFMA call owns all of its scratch: it allocates nothing, and a graph that holds it no buffer of ours
+    ws = workspace(_gemm_workspace_bytes(M, N, K), x.device, st) if (M <= GEMV_MAX_M or a_had is None) else None
     gw = w.c()
     return check(lib.hx_exl3_gemm(y.data_ptr(), x.data_ptr(), C.byref(gw), M, N, K, bits, int(y_fp32), st,
                                   _ptr(a_had), int(mcg), _ptr(ws), ws.numel() if ws is not None else 0),

@@ -134,8 +134,7 @@ def test_mfma_row_tiles_and_k_splits(hx, M, K, N, bits, cb, y_fp32):
 
 @pytest.mark.parametrize("ws_bytes", [0, 64 * 1024, 64 * 1024 + 45 * 8 * 4, None])
 def test_mfma_small_workspace(hx, ws_bytes):
-    """a_had given and no workspace, or one too small for the row sums or the K-split partials: the call does
-    without what does not fit."""
+    """a_had given with no workspace, a small one or one of the queried size: the call needs none and leaves it alone."""
     import ctypes as C
     import torch
     from oracle import oracle as O
@@ -156,6 +155,27 @@ def test_mfma_small_workspace(hx, ws_bytes):
     assert r == hx.HX_GEMM_PATH_MFMA
     assert_close(y.cpu().numpy(), ref, what=f"workspace {ws_bytes}")
     assert bool((ws[n:] == 7).all()) and not bool(ws[:min(n, 64 * 1024)].any())
+
+
+def test_mfma_with_a_had_leaves_the_workspace(hx):
+    """The caller's a_had is all the scratch of an M > 16 call: a workspace that another call in flight may be using
+    (nothing in it is zero here) is neither read nor written."""
+    import ctypes as C
+    import torch
+    from oracle import oracle as O
+    from helios_glm53flash_amd._lib import lib
+    M, K, N, bits = 45, 2048, 256, 4
+    tr, suh, svh = make_linear(23, K, N, bits)
+    x = make_x(24, M, K)
+    w = hx.GroupWords(_dev(tr, torch.int16), _dev(suh), _dev(svh), hx.MUL1)
+    xd, a_had, y = _dev(x), torch.empty((M, K), dtype=torch.float16, device="cuda"), torch.empty((M, N), device="cuda")
+    ws = torch.full((64 << 20,), 5, dtype=torch.uint8, device="cuda")
+    gw = w.c()
+    r = lib.hx_exl3_gemm(y.data_ptr(), xd.data_ptr(), C.byref(gw), M, N, K, bits, 1, None, a_had.data_ptr(), 0,
+                         ws.data_ptr(), ws.numel())
+    torch.cuda.synchronize()
+    assert r == hx.HX_GEMM_PATH_MFMA and bool((ws == 5).all())
+    assert_close(y.cpu().numpy(), O.linear(x, tr, suh, svh, K, N, bits, 2, out_f16=False), what="a_had")
 
 
 def test_gemv_many_splits(hx):

@@ -1,7 +1,8 @@
-"""Host side of the layer calls: the bit widths passed with the expert tables."""
+"""Host side of the calls: the bit widths passed with the expert tables, the workspaces passed to the linear."""
+import pytest
 import torch
 
-from helios_glm53flash_amd import moe
+from helios_glm53flash_amd import exl3, moe
 
 
 def _experts(bits):
@@ -25,3 +26,51 @@ def test_call_bits_with_tables_set_by_a_loader():
     ex = _experts((4, 4))
     ex._tables = object()  # the checkpoint loader builds the tables itself
     assert ex.call_bits() == (4, 4, 4)
+
+
+@pytest.fixture
+def gemm_args(monkeypatch):
+    """exl3.gemm on CPU tensors of K = N = 128, with the library call recorded instead of made and the stream's
+    workspace (stream 7) already there: returns the call's (a_had, workspace, workspace_bytes)."""
+    seen = []
+    real = exl3.lib
+
+    class Lib:
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+        def hx_exl3_gemm(self, *a):
+            seen.append(a[9:10] + a[11:13])
+            return exl3.HX_GEMM_PATH_MFMA
+
+    monkeypatch.setattr(exl3, "lib", Lib())
+    monkeypatch.setattr(exl3, "_need", lambda *a: None)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    ws = torch.zeros(64 << 20, dtype=torch.uint8)
+    monkeypatch.setattr(exl3, "_workspaces", {(0, 7): ws, (None, 7): ws})  # None: the index of a CPU tensor's device
+    w = exl3.GroupWords(torch.zeros((8, 8, 32), dtype=torch.int16), torch.ones(128).half(), torch.ones(128).half(),
+                        exl3.MUL1)
+
+    def call(M, a_had):
+        x, y = torch.zeros((M, 128)).half(), torch.zeros((M, 128))
+        exl3.gemm(y, x, w, M, 128, 128, 2, True, stream=7, a_had=a_had)
+        return seen.pop()
+
+    return call
+
+
+@pytest.mark.parametrize("capturing", [False, True])
+def test_gemm_with_a_had_passes_no_shared_buffer(gemm_args, monkeypatch, capturing):
+    """M > 16 with the caller's a_had: no buffer of the module goes into the call (a captured graph would keep its
+    address past the buffer's replacement), none is allocated and the device is not synchronized."""
+    def refused(*a, **k):
+        raise AssertionError("allocation or synchronisation")
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    monkeypatch.setattr(torch.cuda, "synchronize", refused)
+    a_had = torch.zeros((45, 128)).half()
+    assert gemm_args(45, a_had) == (a_had.data_ptr(), None, 0)
+    ws = exl3._workspaces[0, 7]
+    assert gemm_args(45, None) == (None, ws.data_ptr(), ws.numel())
+    assert gemm_args(3, a_had[:3])[1] == ws.data_ptr()  # the GEMV takes its counters and partials from it
+    exl3._workspaces.clear()
+    assert gemm_args(45, a_had) == (a_had.data_ptr(), None, 0) and not exl3._workspaces
