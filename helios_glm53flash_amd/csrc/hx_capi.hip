@@ -173,21 +173,14 @@ static int decode_checked(int r, void* workspace, hx_stream_t stream)
     return hx_moe_check_status(workspace, stream);
 }
 
-// What a call needs at least (M > 16: nothing but the transformed input, when a_had is null).
-static size_t gemm_min_bytes(int M, int N, int K)
+size_t hx_exl3_gemm_workspace_size(int M, int N, int K)
 {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     if (M <= hx::GEMV_MAX_M) return hx::gemv_workspace_bytes(M, K, N);
     return hx::HX_COUNTER_BYTES + align256((size_t)M * K * sizeof(_Float16));
 }
 
-size_t hx_exl3_gemm_workspace_size(int M, int N, int K)
-{
-    if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const size_t least = gemm_min_bytes(M, N, K);
-    if (M <= hx::GEMV_MAX_M) return least;
-    return least + hx::mfma_rs_bytes(M, K) + hx::mfma_partial_bytes(M, K, N);
-}
+size_t hx_exl3_gemm_extra_bytes(void) { return hx::MFMA_EXTRA_BYTES; }
 
 int hx_exl3_gemm(void* y, const void* x, const hx_group_words* w, int M, int N, int K, int bits, int y_fp32,
                  hx_stream_t stream, void* a_had, int mcg, void* workspace, size_t workspace_bytes)
@@ -222,17 +215,16 @@ int hx_exl3_gemm(void* y, const void* x, const hx_group_words* w, int M, int N, 
     // workspace: such calls need nothing of it, so they may overlap, or sit in a graph that outlives it.
     float* rs = nullptr;
     void* partial = nullptr;
-    size_t o = hx::HX_COUNTER_BYTES + align256((size_t)M * K * sizeof(_Float16));
-    if (!a_had && workspace_bytes >= o + hx::mfma_rs_bytes(M, K)) {
+    const hx::MfmaExtra ex = hx::mfma_extra(M, K, N);
+    const size_t o = hx::HX_COUNTER_BYTES + align256((size_t)M * K * sizeof(_Float16));
+    if (!a_had && ex.rs && workspace_bytes >= o + ex.rs) {
         rs = reinterpret_cast<float*>(static_cast<char*>(workspace) + o);
-        o += hx::mfma_rs_bytes(M, K);
-        const size_t pb = hx::mfma_partial_bytes(M, K, N);
-        if (pb && workspace_bytes >= o + pb) partial = static_cast<char*>(workspace) + o;
+        if (ex.partial && workspace_bytes >= o + ex.rs + ex.partial) partial = static_cast<char*>(workspace) + o + ex.rs;
     }
     int r = hip_status(hx::launch_input_had(xh, suh, ah, rs, M, K, st), "hx_exl3_gemm(input transform)");
     if (r) return r;
-    r = hip_status(hx::launch_linear_mfma(ah, rs, tr, svh, y, M, K, N, bits, cb, y_fp32 != 0, partial,
-                                          static_cast<int*>(workspace), st),
+    r = hip_status(hx::launch_linear_mfma(ah, rs, tr, svh, y, M, K, N, bits, cb, y_fp32 != 0, partial ? ex.splits : 1,
+                                          partial, static_cast<int*>(workspace), st),
                    "hx_exl3_gemm(mfma)");
     return r ? r : HX_GEMM_PATH_MFMA;
 }
@@ -246,12 +238,14 @@ int hx_exl3_gemm(void* y, const void* x, const hx_group_words* w, int M, int N, 
 // the current device, never the array's name (on the host that name is not a device address).  The
 // first HX_COUNTER_BYTES are arrival counters: zero when the code object loads (static storage) and
 // left at zero by every kernel that uses them, so no call clears them; the rest (split-K partials,
-// or the transformed activations of the MFMA path) is written before it is read in every call.
+// or the transformed activations of the MFMA path) is written before it is read in every call.  Calls
+// are accepted by what they need at least; the extra bytes behind it give every accepted shape the path (and the
+// rounding) of hx_exl3_gemm with an ample workspace.
 namespace {
 
 constexpr size_t HX_NOALLOC_SCRATCH_BYTES = 8u << 20;
 constexpr int HX_NOALLOC_MAX_DEVICES = 64;
-__device__ __align__(256) static unsigned char scratch[HX_NOALLOC_SCRATCH_BYTES];
+__device__ __align__(256) static unsigned char scratch[HX_NOALLOC_SCRATCH_BYTES + hx::MFMA_EXTRA_BYTES];
 
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[HX_NOALLOC_MAX_DEVICES];
@@ -283,7 +277,7 @@ int hx_exl3_gemm_noalloc(void* y, const void* x, const hx_group_words* w, int M,
                          hx_stream_t stream, int mcg)
 {
     if (M < 0 || N <= 0 || K <= 0) return fail(HX_ERR_INVALID, "hx_exl3_gemm_noalloc: bad extents");
-    const size_t need = gemm_min_bytes(M, N, K);
+    const size_t need = hx_exl3_gemm_workspace_size(M, N, K);
     if (need > HX_NOALLOC_SCRATCH_BYTES) {
         snprintf(g_err, sizeof(g_err),
                  "hx_exl3_gemm_noalloc: M=%d N=%d K=%d needs %zu bytes of scratch, more than its %zu (use hx_exl3_gemm "
@@ -296,7 +290,7 @@ int hx_exl3_gemm_noalloc(void* y, const void* x, const hx_group_words* w, int M,
         const int r = scratch_ptr(&ws);
         if (r) return r;
     }
-    return hx_exl3_gemm(y, x, w, M, N, K, bits, y_fp32, stream, nullptr, mcg, ws, HX_NOALLOC_SCRATCH_BYTES);
+    return hx_exl3_gemm(y, x, w, M, N, K, bits, y_fp32, stream, nullptr, mcg, ws, sizeof(scratch));
 }
 
 int hx_exl3_reconstruct_slice(void* unpacked, const void* packed, int packed_rows, int packed_cols,

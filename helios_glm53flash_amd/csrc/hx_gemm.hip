@@ -66,7 +66,7 @@ hipError_t launch_input_had(const _Float16* x, const _Float16* suh, _Float16* a,
 // column tiles) at M = 45 / 128: 58 / 67 us unsplit, 35.0 / 49.4 with 2, 28.8 / 42.6 with 4, 27.3 / 41.1 with 5,
 // 28.9 / 49.4 with 8; 24576 columns (192 tiles) at M = 45: 44.6 with 2, 36.5 with 4; 8192 -> 8192 (64 tiles): 63.0
 // with 2, 42.3 with 5, 37.1 with 8 (graphs of 10 calls, input transform included).
-int mfma_splits(int M, int K, int N)
+static int mfma_splits(int M, int K, int N)
 {
     const long tiles = (long)((M + MF_BM - 1) / MF_BM) * (N / 128), nk = K / MF_BK;
     auto least = [](long a, long b) { return a < b ? a : b; };
@@ -77,21 +77,31 @@ int mfma_splits(int M, int K, int N)
 
 static size_t al256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-size_t mfma_rs_bytes(int M, int K) { return al256((size_t)M * (K / 128) * sizeof(float)); }
+// 16-column fragments of accumulators that a split of the tallest row tile stores.
+static int mfma_frags(int M) { return ((M < MF_BM ? M : MF_BM) + 15) / 16 * 2; }
 
-size_t mfma_partial_bytes(int M, int K, int N)
+// A function of the shape alone, so that a shape takes the same path (and rounds alike) wherever MFMA_EXTRA_BYTES are
+// there: what does not fit those is left out even if the caller has more.
+MfmaExtra mfma_extra(int M, int K, int N)
 {
-    const int s = mfma_splits(M, K, N);
-    if (s == 1) return 0;
-    return (size_t)((M + MF_BM - 1) / MF_BM) * (N / 128) * s * MF_BM * 128 * sizeof(float);
+    MfmaExtra e{al256((size_t)M * (K / 128) * sizeof(float)), 0, 1};
+    if (e.rs > MFMA_EXTRA_BYTES) return MfmaExtra{0, 0, 1};
+    const size_t one = (size_t)((M + MF_BM - 1) / MF_BM) * (N / 128) * mfma_frags(M) * MF_THREADS * sizeof(hx_f4);
+    int s = mfma_splits(M, K, N);
+    while (s > 1 && e.rs + s * one > MFMA_EXTRA_BYTES) --s;
+    if (s > 1) {
+        e.partial = s * one;
+        e.splits = s;
+    }
+    return e;
 }
 
 hipError_t launch_linear_mfma(const _Float16* a_had, const float* rs, const uint16_t* trellis, const _Float16* svh,
-                              void* y, int M, int K, int N, int bits, int cb, bool y_fp32, void* partial, int* counter,
-                              hipStream_t st)
+                              void* y, int M, int K, int N, int bits, int cb, bool y_fp32, int splits, void* partial,
+                              int* counter, hipStream_t st)
 {
     MfmaGemmArgs g{a_had, rs, reinterpret_cast<const uint32_t*>(trellis), svh, y, M, K, N, y_fp32,
-                   rs && partial ? mfma_splits(M, K, N) : 1, static_cast<hx_f4*>(partial), counter};
+                   splits, mfma_frags(M), static_cast<hx_f4*>(partial), counter};
     switch (bits) {
         case 1: return launch_mfma_b<1>(cb, g, st);
         case 2: return launch_mfma_b<2>(cb, g, st);

@@ -17,7 +17,8 @@ struct MfmaGemmArgs {
     int M, K, N;
     bool y_fp32;
     int splits;               // K splits (> 1: partial and counter are used, rs is not null)
-    hx_f4* partial;           // [tile][split][BM / 16][2][256] raw accumulators
+    int frags;                // accumulator fragments stored per (tile, split), 2 per 16 rows
+    hx_f4* partial;           // [tile][split][frags][256] raw accumulators
     int* counter;             // [tile]
 };
 
@@ -124,9 +125,9 @@ __device__ __forceinline__ void linear_tile(const MfmaGemmArgs& g, int mt, int c
         if (g.splits > 1) {
             const int tile = mt * (g.N >> 7) + cg;
             constexpr int NF = BM / 16 * 2;
-            const __amdgpu_buffer_rsrc_t rp = mf_rsrc(g.partial + (size_t)tile * g.splits * (MF_BM / 16 * 2) * MF_THREADS,
-                                                      (size_t)g.splits * (MF_BM / 16 * 2) * MF_THREADS * sizeof(hx_f4));
-            auto off = [&](int sp, int f) { return ((sp * (MF_BM / 16 * 2) + f) * MF_THREADS + t) * (int)sizeof(hx_f4); };
+            const __amdgpu_buffer_rsrc_t rp = mf_rsrc(g.partial + (size_t)tile * g.splits * g.frags * MF_THREADS,
+                                                      (size_t)g.splits * g.frags * MF_THREADS * sizeof(hx_f4));
+            auto off = [&](int sp, int f) { return ((sp * g.frags + f) * MF_THREADS + t) * (int)sizeof(hx_f4); };
             const int nf = (rows + 15) / 16 * 2;  // fragments that hold rows
 #pragma unroll
             for (int f = 0; f < NF; ++f)

@@ -53,6 +53,7 @@ def _need(t: torch.Tensor, name: str, dtypes: tuple) -> None:
 
 
 _workspaces: dict[tuple, torch.Tensor] = {}
+_GEMM_EXTRA = lib.hx_exl3_gemm_extra_bytes()
 
 
 def workspace(nbytes: int, device: Optional[torch.device] = None, stream=None) -> torch.Tensor:
@@ -61,7 +62,10 @@ def workspace(nbytes: int, device: Optional[torch.device] = None, stream=None) -
     a time: calls on different streams get different workspaces, so their arrival counters and
     ready flags never meet.  Growing synchronizes the device twice: before the old buffer is
     released (kernels still queued on any stream may use it) and after the zero fill (issued on
-    torch's current stream, the kernels run on `stream`).  Grow outside graph capture."""
+    torch's current stream, the kernels run on `stream`).  Grow outside graph capture.
+    _GEMM_EXTRA bytes follow the nbytes at every size, so the linear finds room for its K splits on any stream
+    that has a workspace at all: they neither make one grow (a graph may hold its address) nor depend on what
+    ran before."""
     if isinstance(device, torch.device):
         dev = device
     else:
@@ -69,12 +73,12 @@ def workspace(nbytes: int, device: Optional[torch.device] = None, stream=None) -
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
     key = (idx, _stream(stream))
     ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
+    if ws is None or ws.numel() - _GEMM_EXTRA < nbytes:
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("the workspace of this stream must be allocated before graph capture: run the call "
                                "once on the capturing stream first, or pass a workspace")
         torch.cuda.synchronize(idx)
-        ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
+        ws = torch.zeros(max(nbytes, 1 << 20) + _GEMM_EXTRA, dtype=torch.uint8, device=dev)
         torch.cuda.synchronize(idx)
         _workspaces[key] = ws
     return ws

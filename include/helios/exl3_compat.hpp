@@ -62,6 +62,8 @@ public:
             if (it->second.bytes < bytes) throw Error("installed workspace is smaller than the call needs");
             return View{it->second.ptr, it->second.bytes};
         }
+        // room for the linear's K splits behind every size, so that they never make a buffer grow
+        const size_t extra = hx_exl3_gemm_extra_bytes();
         Slot& slot = slots_[Key{dev, s}];
         if (slot.bytes < bytes) {
             if (slot.ptr) {
@@ -69,11 +71,11 @@ public:
                 (void)hipFree(slot.ptr);
                 slot = Slot{};
             }
-            if (hipMalloc(&slot.ptr, bytes) != hipSuccess) throw Error("workspace allocation failed");
+            if (hipMalloc(&slot.ptr, bytes + extra) != hipSuccess) throw Error("workspace allocation failed");
             slot.bytes = bytes;
-            check(hx_workspace_init(slot.ptr, bytes, (hx_stream_t)s), "hx_workspace_init");
+            check(hx_workspace_init(slot.ptr, bytes + extra, (hx_stream_t)s), "hx_workspace_init");
         }
-        return View{slot.ptr, slot.bytes};
+        return View{slot.ptr, slot.bytes + extra};
     }
     // Install a caller-owned, zero-filled workspace for every call on the current device; the caller
     // then keeps calls on different streams from overlapping.

@@ -100,18 +100,22 @@ const char* hx_profile_phase_name(int phase);
  * Replaces helios::exl3::gemm (src/cuda/quant/exl3_gemm.cuh:51-66, exl3_gemm.cu:81-243).
  * M <= 16 runs the fused decode-GEMV (returns HX_GEMM_PATH_GEMV), else the MFMA GEMM (returns
  * HX_GEMM_PATH_MFMA), which needs a_had (M*K fp16 scratch, as in the reference; the workspace is then
- * not touched) or, when a_had is NULL, takes it from the workspace (whatever else the queried size holds
- * then, row sums and K-split partials, makes the call faster; it works without).  K % 128 == 0,
- * N % 128 == 0, bits 1..8.  M == 0 is
- * a no-op (x and y may then be NULL). */
+ * not touched) or, when a_had is NULL, takes it from the workspace.  K % 128 == 0, N % 128 == 0,
+ * bits 1..8.  M == 0 is a no-op (x and y may then be NULL).
+ * hx_exl3_gemm_workspace_size is what a call needs.  What the workspace has beyond it makes an M > 16 call with
+ * a_had NULL faster (row sums of the input, K-split partials; the order of the fp32 sums, so the last bits,
+ * change with it): hx_exl3_gemm_extra_bytes() more bytes, a constant of 64 MiB, are enough at every shape, and a
+ * shape then always takes the same path. */
 size_t hx_exl3_gemm_workspace_size(int M, int N, int K);
+size_t hx_exl3_gemm_extra_bytes(void);
 int hx_exl3_gemm(void* y, const void* x, const hx_group_words* w, int M, int N, int K, int bits, int y_fp32,
                  hx_stream_t stream, void* a_had, int mcg, void* workspace, size_t workspace_bytes);
 
 /* hx_exl3_gemm without a workspace argument and without any allocation: the scratch memory (arrival
  * counters, split-K partials, the MFMA path's transformed activations) is a fixed device array of
- * the library, hx_exl3_gemm_noalloc_max_bytes() = 8 MiB per GPU, held until the process ends.
- * Calls whose hx_exl3_gemm_workspace_size(M, N, K) exceeds it return HX_ERR_WORKSPACE.  Every call
+ * the library, hx_exl3_gemm_noalloc_max_bytes() = 8 MiB and hx_exl3_gemm_extra_bytes() per GPU, held until the
+ * process ends; the results are those of hx_exl3_gemm with such a workspace, bit for bit.  Calls whose
+ * hx_exl3_gemm_workspace_size(M, N, K) exceeds the 8 MiB return HX_ERR_WORKSPACE.  Every call
  * on one GPU uses that GPU's array: calls that overlap on one GPU (two streams, two host threads)
  * race.  No counterpart in the reference; it is for callers that cannot allocate, such as code
  * under graph capture or serving loops that forbid hipMalloc. */

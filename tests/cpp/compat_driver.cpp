@@ -248,6 +248,30 @@ int main(int argc, char** argv)
         dump("two_streams_same", &same, sizeof(same));
     }
 
+    // ---- (run in a process of its own) one installed workspace, of the size that the largest M needs
+    if (argc > 2) {
+        const int K = 2048, N = 1024, bits = 2, Mmax = 1024;
+        Lin l(K, N, bits, r);
+        l.dump_as("inst");
+        const size_t bytes = hx_exl3_gemm_workspace_size(Mmax, N, K);
+        void* ws = nullptr;
+        hip_ok(hipMalloc(&ws, bytes), "hipMalloc");
+        hip_ok(hipMemset(ws, 0, bytes), "memset");
+        helios::exl3::set_workspace(ws, bytes);
+        for (int M : {Mmax, 512, 45, 17}) {
+            const auto x = normal_f16((size_t)M * K, r);
+            uint16_t* dx = upload(x);
+            float* y = nullptr;
+            hip_ok(hipMalloc(&y, (size_t)M * N * 4), "hipMalloc");
+            helios::exl3::gemm(y, dx, l.gw(), M, N, K, bits, true, s);
+            hip_ok(hipStreamSynchronize(s), "sync");
+            const auto hy = download(y, (size_t)M * N);
+            dump(("inst_m" + std::to_string(M) + "_x").c_str(), x.data(), x.size() * 2);
+            dump(("inst_m" + std::to_string(M) + "_y").c_str(), hy.data(), hy.size() * 4);
+        }
+        return 0;
+    }
+
     // ---- the engine's routed-MoE sequence (runner.cpp:759-764, 918-922): router, permutation,
     //      moe_grouped with sorted contributions, ordered reduction; then the dense fallback's row glue
     const int E = 16, hidden = 512, inter = 256, topk = 4, bits = 2;

@@ -143,3 +143,23 @@ def test_compat_host_cost(run):
     t = timing["host_us_per_call"]
     print("host us per call:", t)
     assert t["moe_layer_config3"] < 10.0 and t["gemm_config1"] < 10.0
+
+
+def test_compat_one_installed_workspace(tmp_path):
+    """set_workspace with the size of the largest M: smaller M are accepted with it."""
+    import torch
+    from oracle import oracle as O
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    r = subprocess.run([str(DRIVER), str(tmp_path), "installed"], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+    def load(name, dtype):
+        return np.fromfile(tmp_path / f"{name}.bin", dtype=dtype)
+    K, N, bits = 2048, 1024, 2
+    tr, suh, svh = _lin(load, "inst")
+    tr = tr.reshape(K // 16, N // 16, 16 * bits)
+    for M in (512, 45, 17):
+        x = load(f"inst_m{M}_x", np.uint16).reshape(M, K)
+        y = load(f"inst_m{M}_y", np.float32).reshape(M, N)
+        assert_close(y, O.linear(x, tr, suh, svh, K, N, bits, 2), what=f"installed workspace, M={M}")

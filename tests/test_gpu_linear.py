@@ -157,6 +157,72 @@ def test_mfma_small_workspace(hx, ws_bytes):
     assert bool((ws[n:] == 7).all()) and not bool(ws[:min(n, 64 * 1024)].any())
 
 
+@pytest.mark.parametrize("M,N", [(45, 512), (300, 256)])
+def test_mfma_workspace_beyond_the_least(hx, M, N):
+    """Without a_had: the least workspace, room for the row sums, one byte short of the K-split partials, and enough
+    for them.  Nothing past the end is written, the counters return to zero."""
+    import ctypes as C
+    import torch
+    from oracle import oracle as O
+    from helios_glm53flash_amd._lib import HX_ERR_WORKSPACE, lib
+    K, bits = 2048, 4
+    tr, suh, svh = make_linear(31, K, N, bits)
+    x = make_x(32, M, K)
+    w = hx.GroupWords(_dev(tr, torch.int16), _dev(suh), _dev(svh), hx.MUL1)
+    ref = O.linear(x, tr, suh, svh, K, N, bits, 2, out_f16=False)
+    xd, gw = _dev(x), w.c()
+    least = lib.hx_exl3_gemm_workspace_size(M, N, K)
+    rs = (M * K // 32 + 255) // 256 * 256  # an fp32 sum per 128 inputs
+    # 2048 / 64 = 32 chunks of k: 4 splits of 8; a split stores 16-row fragments of 128 columns, a row tile at most 128 rows
+    partial = (M + 127) // 128 * (N // 128) * 4 * ((min(M, 128) + 15) // 16 * 16) * 128 * 4
+    outs = []
+    for n in (least, least + rs, least + rs + partial - 1, least + rs + partial,
+              least + lib.hx_exl3_gemm_extra_bytes()):
+        ws = torch.zeros(n + 4096, dtype=torch.uint8, device="cuda")
+        ws[n:] = 7
+        y = torch.empty((M, N), device="cuda")
+        r = lib.hx_exl3_gemm(y.data_ptr(), xd.data_ptr(), C.byref(gw), M, N, K, bits, 1, None, None, 0, ws.data_ptr(), n)
+        torch.cuda.synchronize()
+        assert r == hx.HX_GEMM_PATH_MFMA
+        assert_close(y.cpu().numpy(), ref, what=f"workspace of {n}")
+        assert bool((ws[n:] == 7).all()) and not bool(ws[:64 * 1024].any())
+        outs.append(y)
+    assert torch.equal(outs[1], outs[2]) and torch.equal(outs[3], outs[4]) and not torch.equal(outs[2], outs[3])
+    ws = torch.zeros(least, dtype=torch.uint8, device="cuda")
+    assert lib.hx_exl3_gemm(outs[0].data_ptr(), xd.data_ptr(), C.byref(gw), M, N, K, bits, 1, None, None, 0,
+                            ws.data_ptr(), 64 * 1024) == HX_ERR_WORKSPACE
+
+
+def test_mfma_captured_on_a_decode_stream(hx):
+    """An M > 16 linear captured on a stream that only ran M = 1: every replay gives the eager bits, also after eager
+    calls of other shapes on the stream, which must not move or release the workspace that the graph holds."""
+    import torch
+    K, N, bits = 4096, 1024, 4
+    tr, suh, svh = make_linear(41, K, N, bits)
+    w = hx.GroupWords(_dev(tr, torch.int16), _dev(suh), _dev(svh), hx.MUL1)
+    x = {M: _dev(make_x(42 + M, M, K)) for M in (1, 45, 100)}
+    y = {M: torch.empty((M, N), device="cuda") for M in x}
+    eager = torch.empty((45, N), device="cuda")
+    hx.gemm(eager, x[45], w, 45, N, K, bits, True)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    hx.gemm(y[1], x[1], w, 1, N, K, bits, True, stream=s)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        hx.gemm(y[45], x[45], w, 45, N, K, bits, True)
+    for rep in range(4):
+        y[45].fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y[45], eager), rep
+        hx.gemm(y[100], x[100], w, 100, N, K, bits, True, stream=s)  # eager work between replays
+        torch.full((1 << 20,), -1.0, device="cuda")
+        torch.cuda.synchronize()
+
+
 def test_mfma_with_a_had_leaves_the_workspace(hx):
     """The caller's a_had is all the scratch of an M > 16 call: a workspace that another call in flight may be using
     (nothing in it is zero here) is neither read nor written."""

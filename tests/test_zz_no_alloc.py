@@ -27,7 +27,8 @@ def _dev(a, dtype=None):
 
 
 @pytest.mark.parametrize("shapes", [((8, 4096, 12288, 4), (1, 4096, 2048, 2)),    # GEMV, split-K partials
-                                    ((200, 2048, 1024, 3), (40, 1024, 512, 2))])  # MFMA, staged activations
+                                    ((200, 2048, 1024, 3), (40, 1024, 512, 2)),   # MFMA, staged activations
+                                    ((128, 4096, 12288, 2), (45, 4096, 2048, 4))])  # K splits of 30 MB, 4 MB
 def test_noalloc_equals_workspace_path(hx, shapes):
     import torch
     for i, (M, K, N, bits) in enumerate(shapes):
