@@ -224,14 +224,20 @@ __device__ __forceinline__ void mfma_tile_q(const _Float16* A, long lda, int row
         else quarter_decode<BITS, CB>(wv[slot], d);
     };
 
+    // VMEM instructions per chunk: A (DMA) and trellis words.  The waits for a chunk's A count whole chunks issued after
+    // it, so a chunk's loads must not move past another chunk's, nor be dropped as unused: the chunks' loads are
+    // kept apart by compiler fences (the steps' by their barriers; within a chunk the order is free), and the
+    // last steps, whose prefetches nothing would read, issue none and wait for what is left.
+    constexpr int NT = quarter_buf_vmem(BITS);  // load_t = one load_quarter_buf
+    constexpr int NCHUNK = NA + NT;
+    static_assert(!DMA || (PF - 1) * NCHUNK < 64, "vmcnt range");
     const int nk = K / MF_BK;
 #pragma unroll
-    for (int s = 0; s < (PF > PT ? PF : PT); ++s) {
-        if (s < PF) {
-            if constexpr (DMA) load_a_lds(s, min(s, nk - 1) * MF_BK);
-            else load_a(s, min(s, nk - 1) * MF_BK);
-        }
-        if (s < PT) load_t(s, min(s, nk - 1) * MF_BK);
+    for (int s = 0; s < PF; ++s) {
+        if constexpr (DMA) load_a_lds(s, min(s, nk - 1) * MF_BK);
+        else load_a(s, min(s, nk - 1) * MF_BK);
+        load_t(s, min(s, nk - 1) * MF_BK);
+        asm volatile("" ::: "memory");
     }
     // row t's precomputed sum, requested while the first chunks are in flight (32 independent
     // loads per round trip: one round trip for K up to 4096)
@@ -246,14 +252,8 @@ __device__ __forceinline__ void mfma_tile_q(const _Float16* A, long lda, int row
                 for (int j = 0; j < 32; ++j) rs_ext += v[j];
             }
     }
-    // VMEM instructions per chunk: A (DMA) and trellis words; chunk c + 1's A is complete once at
-    // most the loads of the PF - 1 later chunks are outstanding (their order within a step is left
-    // to the compiler, so the count takes whole chunks)
-    constexpr int NT = quarter_buf_vmem(BITS);  // load_t = one load_quarter_buf
-    constexpr int A_WAIT = (PF - 1) * (NA + NT);
-    static_assert(!DMA || A_WAIT < 64, "vmcnt range");
-    // chunk 0: the prologue issued at most the other chunks' loads after it
-    if constexpr (DMA) __builtin_amdgcn_s_waitcnt(qt_vmcnt((PF - 1) * NA + (PT - 1) * NT));
+    // chunk 0: the loads of the PF - 1 chunks behind it may be outstanding
+    if constexpr (DMA) __builtin_amdgcn_s_waitcnt(qt_vmcnt((PF - 1) * NCHUNK));
     else store_a(0, 0, true);
     // d holds the decoded quarter of the current chunk; the next chunk's quarter is decoded into it
     // after the chunk's MFMAs (their B operands are read before the decode overwrites it)
@@ -261,12 +261,16 @@ __device__ __forceinline__ void mfma_tile_q(const _Float16* A, long lda, int row
     uint32_t d[ND][16];
     decode(0, d[0]);
     hx_lds_barrier();
-    // step c: ua = c % PF, ut = c % PT, par = c & 1, all compile-time in the unrolled loops
-    auto step = [&](int c, auto ua_, auto ut_, auto par_) {
+    // step c: ua = c % PF, ut = c % PT, par = c & 1, all compile-time in the unrolled loops; left < 0: the step requests
+    // chunk c + PF; left >= 0: no loads, and that many chunks behind c + 1 are in flight
+    auto step = [&](int c, auto ua_, auto ut_, auto par_, auto left_) {
         constexpr int ua = decltype(ua_)::value, ut = decltype(ut_)::value, par = decltype(par_)::value;
-        if constexpr (DMA) load_a_lds((c + PF) % NB, min(c + PF, nk - 1) * MF_BK);
-        else load_a(ua, min(c + PF, nk - 1) * MF_BK);
-        load_t(ut, min(c + PT, nk - 1) * MF_BK);
+        constexpr int left = decltype(left_)::value;
+        if constexpr (left < 0) {
+            if constexpr (DMA) load_a_lds((c + PF) % NB, min(c + PF, nk - 1) * MF_BK);
+            else load_a(ua, min(c + PF, nk - 1) * MF_BK);
+            load_t(ut, min(c + PT, nk - 1) * MF_BK);
+        }
         const _Float16* as = a_buf(c % NB);
         const uint32_t* dc = d[par % ND];
         uint32_t* dn = d[(par + 1) % ND];
@@ -291,22 +295,24 @@ __device__ __forceinline__ void mfma_tile_q(const _Float16* A, long lda, int row
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) mfma_rb(rb);
         decode((ut + 1) % PT, dn);
-        if constexpr (DMA) __builtin_amdgcn_s_waitcnt(qt_vmcnt(A_WAIT));
+        if constexpr (DMA) __builtin_amdgcn_s_waitcnt(qt_vmcnt((left < 0 ? PF - 1 : left) * NCHUNK));
         else store_a((ua + 1) % PF, (c + 1) & 1, c + 1 < nk);
         hx_lds_barrier();
     };
     // unrolled period: every ring position and the parity are compile-time constants
     constexpr int PER = qt_lcm(qt_lcm(PF, PT), 2);
+    static_assert(PER == PF, "the last PER - 1 steps read chunks that are all in flight before them");
     const int nmain = nk - nk % PER;
     for (int c0 = 0; c0 < nmain; c0 += PER) {
         [&]<int... U>(std::integer_sequence<int, U...>) {
             (step(c0 + U, std::integral_constant<int, U % PF>{}, std::integral_constant<int, U % PT>{},
-                  std::integral_constant<int, U & 1>{}), ...);
+                  std::integral_constant<int, U & 1>{}, std::integral_constant<int, -1>{}), ...);
         }(std::make_integer_sequence<int, PER>{});
     }
     [&]<int... U>(std::integer_sequence<int, U...>) {
         ((nmain + U < nk ? step(nmain + U, std::integral_constant<int, U % PF>{},
-                                std::integral_constant<int, U % PT>{}, std::integral_constant<int, U & 1>{})
+                                std::integral_constant<int, U % PT>{}, std::integral_constant<int, U & 1>{},
+                                std::integral_constant<int, (PF - 2 - U > 0 ? PF - 2 - U : 0)>{})
                          : void()), ...);
     }(std::make_integer_sequence<int, PER - 1>{});
     if constexpr (DMA) {

@@ -382,3 +382,34 @@ def test_decode_several_tokens(hx, T, topk, E, hidden, inter, bias):
     per column group, more experts than the parked tables hold, repeated calls on one workspace."""
     for seed in (31, 32):
         _run_layer(hx, E, hidden, inter, topk, T, 2, (2, 3, 2), seed=seed + T + E, bias=bias)
+
+
+@pytest.mark.parametrize("T,topk,bits,shared_bits", [(9, 3, 4, (4, 1, 8)), (40, 4, (5, 2, 3), (2, 2, 2)),
+                                                     (70, 2, (2, 8, 6), (3, 5, 7)), (129, 4, 4, (6, 7, 3))])
+@pytest.mark.parametrize("hidden,inter", [(384, 256), (512, 640)])
+@pytest.mark.parametrize("mcg", [True, False])
+def test_prefill_shared_expert_repeats(hx, T, topk, bits, shared_bits, hidden, inter, mcg):
+    """Both codebooks with a shared expert, every height of its last row tile, chunk counts that end within and with a
+    round of the tiles' rings: the oracle's values, and the same bits at every call (a chunk read before it has
+    arrived would give what the LDS held before)."""
+    import torch
+    from oracle import oracle as O
+    exl3, moe = hx
+    E = 12
+    ex = moe.ExpertSet.synthetic(E, hidden, inter, bits, seed=T + inter, mul1=not mcg)
+    sh = [exl3.GroupWords(w.trellis, w.suh, w.svh, 0 if mcg else exl3.MUL1)
+          for w in moe.synthetic_dense_mlp(hidden, inter, shared_bits, seed=T)]
+    layer = moe.MoeLayer(ex, sh, topk=topk, mcg=mcg)
+    r = np.random.default_rng(T)
+    x = r.standard_normal((T, hidden)).astype(np.float16)
+    scores = r.standard_normal((T, E)).astype(np.float16)
+    xd, sd = torch.from_numpy(x).cuda(), torch.from_numpy(scores).cuda()
+    y_routed = torch.empty((T, hidden), dtype=torch.float32, device="cuda")
+    y = layer(xd, sd, y_routed=y_routed).clone()
+    idx, w = O.routing(scores, topk, 2.5)
+    yr_ref, yo_ref = O.moe_rows(x, hidden, inter, idx, w, np.arange(T), _oracle_experts(ex, set(range(E))),
+                                _oracle_shared(sh), 10.0, cb=1 if mcg else 2)
+    assert_close(y_routed.cpu().numpy(), yr_ref, what=f"routed mcg={mcg} T={T}")
+    assert_close(y.float().cpu().numpy(), yo_ref.view(np.float16).astype(np.float64), what=f"y mcg={mcg} T={T}")
+    for _ in range(10):
+        assert torch.equal(layer(xd, sd), y)
