@@ -66,12 +66,19 @@ hipError_t launch_input_had(const _Float16* x, const _Float16* suh, _Float16* a,
 // column tiles) at M = 45 / 128: 58 / 67 us unsplit, 35.0 / 49.4 with 2, 28.8 / 42.6 with 4, 27.3 / 41.1 with 5,
 // 28.9 / 49.4 with 8; 24576 columns (192 tiles) at M = 45: 44.6 with 2, 36.5 with 4; 8192 -> 8192 (64 tiles): 63.0
 // with 2, 42.3 with 5, 37.1 with 8 (graphs of 10 calls, input transform included).
+// Where tiles alone reach more than half of the CUs a split saves less of a chunk's time, so it has to be longer to
+// be worth its trip: 16 chunks (12 at up to 32 rows, whose accumulators are few), and 24 with more tiles than CUs.
+// 4-bit, 126 rows, 17792 columns (139 tiles), unsplit / 2 splits: K = 1024 25.4 / 30.6 us, K = 1280 29.1 / 32.9,
+// K = 1536 32.8 / 35.6, K = 2048 40.8 / 40.4; 200 rows (278 tiles): K = 1024 28.9 / 36.5, K = 2048 49.5 / 48.4, K = 3072
+// 69.0 / 60.1.  (512 to 24576 columns, K = 512 to 8192, 17 to 512 rows, 2, 4 and 6 bits: no shape more than 2 %
+// slower than unsplit; with 8 chunks everywhere up to 30 %.)
 static int mfma_splits(int M, int K, int N)
 {
     const long tiles = (long)((M + MF_BM - 1) / MF_BM) * (N / 128), nk = K / MF_BK;
     auto least = [](long a, long b) { return a < b ? a : b; };
     const long two = 2 * GEMV_CUS / tiles;
-    const long s = least(least(3 * GEMV_CUS / tiles, two > 5 ? two : 5), least(nk / 8, 8));
+    const long chunks = tiles <= GEMV_CUS / 2 ? 8 : tiles > GEMV_CUS ? 24 : M <= 32 ? 12 : 16;
+    const long s = least(least(3 * GEMV_CUS / tiles, two > 5 ? two : 5), least(nk / chunks, 8));
     return s > 1 ? (int)s : 1;
 }
 

@@ -193,6 +193,30 @@ def test_mfma_workspace_beyond_the_least(hx, M, N):
                             ws.data_ptr(), 64 * 1024) == HX_ERR_WORKSPACE
 
 
+@pytest.mark.parametrize("M,K,N,split", [(126, 1280, 17792, False), (512, 1024, 8192, False), (200, 2048, 17792, False),
+                                         (17, 1280, 24576, False), (126, 1280, 8192, True), (17, 1536, 17792, True),
+                                         (126, 2048, 17792, True), (384, 3072, 12288, True)])
+def test_mfma_splits_only_where_they_pay(hx, M, K, N, split):
+    """Tiles on more than half of the CUs are split only if a split is long enough (shorter ones were up to 30 % slower
+    than no split): with room for the row sums alone the call is unsplit, with more room it is split or the same."""
+    import ctypes as C
+    import torch
+    from helios_glm53flash_amd._lib import lib
+    tr, suh, svh = make_linear(51, K, N, 2)
+    w = hx.GroupWords(_dev(tr, torch.int16), _dev(suh), _dev(svh), hx.MUL1)
+    xd, gw = _dev(make_x(52, M, K)), w.c()
+    least = lib.hx_exl3_gemm_workspace_size(M, N, K)
+    ys = []
+    for n in (least + (M * K // 32 + 255) // 256 * 256, least + lib.hx_exl3_gemm_extra_bytes()):
+        ws = torch.zeros(n, dtype=torch.uint8, device="cuda")
+        y = torch.empty((M, N), device="cuda")
+        lib.hx_exl3_gemm(y.data_ptr(), xd.data_ptr(), C.byref(gw), M, N, K, 2, 1, None, None, 0, ws.data_ptr(), n)
+        torch.cuda.synchronize()
+        ys.append(y)
+    assert torch.equal(*ys) == (not split)
+    assert float((ys[0] - ys[1]).norm() / ys[0].norm()) < 1e-5  # the order of fp32 sums: sqrt(K) * 2^-24 = 4e-6 of the size
+
+
 def test_mfma_captured_on_a_decode_stream(hx):
     """An M > 16 linear captured on a stream that only ran M = 1: every replay gives the eager bits, also after eager
     calls of other shapes on the stream, which must not move or release the workspace that the graph holds."""
