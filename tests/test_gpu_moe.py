@@ -413,3 +413,11 @@ def test_prefill_shared_expert_repeats(hx, T, topk, bits, shared_bits, hidden, i
     assert_close(y.float().cpu().numpy(), yo_ref.view(np.float16).astype(np.float64), what=f"y mcg={mcg} T={T}")
     for _ in range(10):
         assert torch.equal(layer(xd, sd), y)
+
+
+@pytest.mark.parametrize("T,topk,E,hidden,inter", [(2, 8, 24, 4096, 128), (3, 4, 16, 2048, 128), (4, 2, 8, 1152, 256),
+                                                   (5, 2, 9, 4096, 128), (8, 1, 4, 7168, 128)])
+def test_decode_few_column_groups(hx, T, topk, E, hidden, inter):
+    """Phases of few column groups: 3 to 8 units per group, k ranges of unequal length among them."""
+    for _ in range(2):
+        _run_layer(hx, E, hidden, inter, topk, T, 2, 2, seed=T + hidden)
