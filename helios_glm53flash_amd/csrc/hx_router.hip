@@ -81,7 +81,9 @@ __global__ __launch_bounds__(256) void gemv_nt_kernel(const _Float16* x, const _
 // per CU, the 64-byte halves that fragments loaded straight into MFMA layout touch at 37 GB/s (that
 // variant of this kernel: 45 us at M = 4096, 17 us at M = 33-512).
 // LDS rows are 64 halves with the 16-byte chunks of row r permuted by mf_swz(r) (hx_mfma.hpp).
-template <int RB, int CB, int KS, int NB>
+// DMA false: x or w is not 16-byte aligned, which the buffer loads into LDS ask for; the chunks go through
+// registers (global loads take any address), without loads in flight across chunks.
+template <int RB, int CB, int KS, int NB, bool DMA>
 __device__ __forceinline__ void gemm_nt_split(const _Float16* x, const _Float16* w, void* y, int M, int N, int K,
                                               bool y_fp32, bool add)
 {
@@ -107,11 +109,24 @@ __device__ __forceinline__ void gemm_nt_split(const _Float16* x, const _Float16*
     auto load = [&](int p) {
         const int q = q0 + p;
         _Float16* d = wb + p % NB * ROWS * 64;
+        if constexpr (DMA) {
 #pragma unroll
-        for (int i = 0; i < NL; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(i < 2 * RB ? rx : rw,
-                                                     (__attribute__((address_space(3))) void*)(d + 512 * i), 16,
-                                                     voff[i], q * 128, 0, 0);
+            for (int i = 0; i < NL; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(i < 2 * RB ? rx : rw,
+                                                         (__attribute__((address_space(3))) void*)(d + 512 * i), 16,
+                                                         voff[i], q * 128, 0, 0);
+        } else {
+            typedef _Float16 h8a2 __attribute__((ext_vector_type(8), aligned(2)));
+            hx_h8 v[NL];
+#pragma unroll
+            for (int i = 0; i < NL; ++i) {
+                const _Float16* s = (i < 2 * RB ? x + (size_t)r0 * K : w + (size_t)c0 * K) + voff[i] / 2 + 64 * q;
+                v[i] = hx_h8{};
+                if (64 * q + 8 * ((lane & 7) ^ mf_swz(8 * i + (lane >> 3))) < K) v[i] = *reinterpret_cast<const h8a2*>(s);
+            }
+#pragma unroll
+            for (int i = 0; i < NL; ++i) *reinterpret_cast<hx_h8*>(d + 512 * i + 8 * lane) = v[i];
+        }
     };
     hx_f4 acc[RB][CB];
 #pragma unroll
@@ -119,8 +134,10 @@ __device__ __forceinline__ void gemm_nt_split(const _Float16* x, const _Float16*
 #pragma unroll
         for (int j = 0; j < CB; ++j) acc[i][j] = hx_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int p = 0; p < NB; ++p)
+    for (int p = 0; p < NB; ++p) {
         if (p < n) load(p);
+        asm volatile("" ::: "memory");  // the waits below count whole chunks: their loads stay apart
+    }
     for (int p = 0; p < n; ++p) {
         // chunk p has arrived once at most the loads of the later chunks in flight are outstanding
         asm volatile("" ::: "memory");
@@ -182,11 +199,11 @@ __device__ __forceinline__ void gemm_nt_split(const _Float16* x, const _Float16*
             }
 }
 
-template <int RB, int CB, int KS, int NB>
+template <int RB, int CB, int KS, int NB, bool DMA>
 __global__ __launch_bounds__(64 * KS) void gemm_nt_split_kernel(const _Float16* x, const _Float16* w, void* y, int M,
                                                                 int N, int K, bool y_fp32, bool add)
 {
-    gemm_nt_split<RB, CB, KS, NB>(x, w, y, M, N, K, y_fp32, add);
+    gemm_nt_split<RB, CB, KS, NB, DMA>(x, w, y, M, N, K, y_fp32, add);
 }
 
 struct NtCall {
@@ -204,11 +221,11 @@ static long nt_cost(const NtCall& c)
     return (wgs + 255) / 256 * (RB + CB);
 }
 
-template <int RB, int CB, int KS, int NB>
+template <int RB, int CB, int KS, int NB, bool DMA = true>
 static hipError_t nt_launch(const NtCall& c, hipStream_t st)
 {
     constexpr size_t lds = sizeof(_Float16) * KS * NB * 16 * (RB + CB) * 64;
-    hipLaunchKernelGGL((gemm_nt_split_kernel<RB, CB, KS, NB>),
+    hipLaunchKernelGGL((gemm_nt_split_kernel<RB, CB, KS, NB, DMA>),
                        dim3((c.M + 16 * RB - 1) / (16 * RB), (c.N + 16 * CB - 1) / (16 * CB)), dim3(64 * KS), lds, st,
                        c.x, c.w, c.y, c.M, c.N, c.K, c.y_fp32, c.add);
     return hipGetLastError();
@@ -227,6 +244,7 @@ hipError_t launch_gemm_nt_f16(const _Float16* x, const _Float16* w, void* y, int
         // The tile with the least reading on the busiest CU; equal costs go to the larger tile (fewer bytes
         // in all).
         const NtCall c{x, w, y, M, N, K, y_fp32, add};
+        if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) return nt_launch<2, 2, 8, 2, false>(c, st);
         const long cost[5] = {nt_cost<4, 6>(c), nt_cost<4, 4>(c), nt_cost<2, 3>(c), nt_cost<2, 2>(c), nt_cost<1, 1>(c)};
         int best = 0;
         for (int i = 1; i < 5; ++i)

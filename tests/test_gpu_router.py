@@ -135,3 +135,28 @@ def test_gemm_nt_split_tiles(M, N, K, add):
     exl3.gemm_nt_f16(y, x, w, M, N, K, y_fp32=True, add=add)
     torch.cuda.synchronize()
     assert float((y.double() - ref).abs().max()) <= 1e-5 * K ** 0.5 * 5
+
+
+@pytest.mark.parametrize("M,N,K,xoff,woff", [
+    (4090, 160, 1056, 0, 0), (3001, 150, 96, 0, 0),                       # the 64 x 64 tile
+    (100, 72, 2016, 1, 0), (33, 288, 4096, 0, 1), (17, 40, 96, 2, 4),     # operands off a 16-byte boundary by
+    (70, 64, 32, 4, 2), (2100, 288, 544, 3, 5), (5, 160, 4096, 1, 1)])    # an odd and an even number of elements
+def test_gemm_nt_tiles_and_alignment(M, N, K, xoff, woff):
+    """Contiguous views that start anywhere in their storage; the elements around them are NaN.  The bound is that of
+    the tile test above."""
+    import torch
+    from helios_glm53flash_amd import exl3
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + N + K)
+
+    def view(rows, off):
+        buf = torch.full((rows * K + 16,), float("nan"), dtype=torch.float16, device="cuda")
+        v = buf[off:off + rows * K].view(rows, K)
+        v.copy_(torch.randn((rows, K), generator=g, device="cuda"))
+        return v
+    x, w = view(M, xoff), view(N, woff)
+    assert x.is_contiguous() and x.data_ptr() % 16 == 2 * xoff and w.data_ptr() % 16 == 2 * woff
+    y = torch.empty((M, N), device="cuda")
+    exl3.gemm_nt_f16(y, x, w, M, N, K, y_fp32=True)
+    torch.cuda.synchronize()
+    assert float((y.double() - x.double() @ w.double().T).abs().max()) <= 1e-5 * K ** 0.5 * 5
