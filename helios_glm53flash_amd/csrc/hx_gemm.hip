@@ -7,45 +7,46 @@ namespace hx {
 template <int BITS>
 hipError_t launch_mfma_b(int cb, const MfmaGemmArgs& g, hipStream_t st);  // hx_gemm_b*.hip
 
-// a = fp16(H128(fp16(x . suh))) row-wise (had_hf_r_128_inner<true,false>) and, with rs, the fp32 sum of each
+// a = fp16(H128(fp16(x . suh))) row-wise (had_hf_r_128_inner<true,false>) and, with RS, the fp32 sum of each
 // 128-wide block of a.  One wave per 16 consecutive blocks on the matrix cores (hx_gemv.hpp), the
 // results stored 16 bytes per lane through LDS.  Bound: memory; M = 2000, K = 4096 (33 MB) 15.6 us with
-// one block per wave and a shuffle butterfly.
+// one block per wave and a shuffle butterfly.  Few rows: latency, so the column of a block comes from a 32-bit
+// remainder (a 64-bit one is a hundred instructions ahead of the first load) and sums nobody reads are not made.
 constexpr int HAD_LD = 128 + 8;  // halves per staged block
+template <bool RS>
 __global__ __launch_bounds__(256) void input_had_kernel(const _Float16* x, const _Float16* suh, _Float16* a, float* rs,
-                                                        long blocks, int nblk)
+                                                        uint32_t blocks, uint32_t nblk)
 {
     __shared__ _Float16 stage[4][16 * HAD_LD];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long b0 = ((long)blockIdx.x * 4 + wave) * 16;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t b0 = (blockIdx.x * 4 + wave) * 16;
     if (b0 >= blocks) return;
-    const int g = lane >> 4;
-    const long b = min(b0 + (lane & 15), blocks - 1);
-    const _Float16* xb = x + b * 128 + 8 * g;
+    const uint32_t g = lane >> 4;
+    const uint32_t b = min(b0 + (lane & 15), blocks - 1);
+    const _Float16* xb = x + (size_t)b * 128 + 8 * g;
     const _Float16* sb = suh + (b % nblk) * 128 + 8 * g;
     InputRegs r;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-        r.x[kk] = *reinterpret_cast<const hx_h8u*>(xb + 32 * kk);
-        r.s[kk] = *reinterpret_cast<const hx_h8u*>(sb + 32 * kk);
-    }
+    for (int kk = 0; kk < 4; ++kk) r.x[kk] = *reinterpret_cast<const hx_h8u*>(xb + 32 * kk);
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) r.s[kk] = *reinterpret_cast<const hx_h8u*>(sb + 32 * kk);
     _Float16* sw = stage[wave];
     input_store(reinterpret_cast<uint32_t*>(sw), r, 16, 0, HAD_LD);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int j = 4 * q + g, c8 = 8 * (lane & 15);
+    for (uint32_t q = 0; q < 4; ++q) {
+        const uint32_t j = 4 * q + g, c8 = 8 * (lane & 15);
         const hx_h8 v = *reinterpret_cast<const hx_h8*>(sw + j * HAD_LD + c8);
-        float s = 0.0f;
+        if (b0 + j < blocks) *reinterpret_cast<hx_h8u*>(a + (size_t)(b0 + j) * 128 + c8) = v;
+        if constexpr (RS) {
+            float s = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) s += (float)v[i];
+            for (int i = 0; i < 8; ++i) s += (float)v[i];
 #pragma unroll
-        for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 64);
-        if (b0 + j < blocks) {
-            *reinterpret_cast<hx_h8u*>(a + (b0 + j) * 128 + c8) = v;
-            if (rs && (lane & 15) == 0) rs[b0 + j] = s;
+            for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 64);
+            if (b0 + j < blocks && (lane & 15) == 0) rs[b0 + j] = s;
         }
     }
 }
@@ -53,10 +54,11 @@ __global__ __launch_bounds__(256) void input_had_kernel(const _Float16* x, const
 hipError_t launch_input_had(const _Float16* x, const _Float16* suh, _Float16* a, float* rs, long rows, int K,
                             hipStream_t st)
 {
-    const long blocks = rows * (K / 128);
+    const long blocks = rows * (K / 128);  // of 128 fp16: 2^32 of them would be 1 TiB
     if (blocks == 0) return hipSuccess;
-    hipLaunchKernelGGL(input_had_kernel, dim3((unsigned)((blocks + 63) / 64)), dim3(256), 0, st, x, suh, a, rs, blocks,
-                       K / 128);
+    if (blocks > 0xffffffffl - 64) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((rs ? input_had_kernel<true> : input_had_kernel<false>), dim3((unsigned)((blocks + 63) / 64)),
+                       dim3(256), 0, st, x, suh, a, rs, (uint32_t)blocks, (uint32_t)(K / 128));
     return hipGetLastError();
 }
 
