@@ -213,18 +213,15 @@ int hx_exl3_gemm(void* y, const void* x, const hx_group_words* w, int M, int N, 
     // Row sums of the transformed input and K-split partials go to what the workspace has beyond the counters and
     // the transformed input; a smaller workspace does without them.  A call with its own a_had does not touch the
     // workspace: such calls need nothing of it, so they may overlap, or sit in a graph that outlives it.
-    float* rs = nullptr;
-    void* partial = nullptr;
-    const hx::MfmaExtra ex = hx::mfma_extra(M, K, N);
     const size_t o = hx::HX_COUNTER_BYTES + align256((size_t)M * K * sizeof(_Float16));
-    if (!a_had && ex.rs && workspace_bytes >= o + ex.rs) {
-        rs = reinterpret_cast<float*>(static_cast<char*>(workspace) + o);
-        if (ex.partial && workspace_bytes >= o + ex.rs + ex.partial) partial = static_cast<char*>(workspace) + o + ex.rs;
-    }
+    hx::MfmaExtra ex = hx::mfma_extra(M, K, N, bits, cb);
+    if (a_had || workspace_bytes < o + ex.rs + ex.partial) ex = hx::MfmaExtra{0, 0, 1};
+    float* rs = ex.rs ? reinterpret_cast<float*>(static_cast<char*>(workspace) + o) : nullptr;
+    void* partial = ex.partial ? static_cast<char*>(workspace) + o + ex.rs : nullptr;
     int r = hip_status(hx::launch_input_had(xh, suh, ah, rs, M, K, st), "hx_exl3_gemm(input transform)");
     if (r) return r;
-    r = hip_status(hx::launch_linear_mfma(ah, rs, tr, svh, y, M, K, N, bits, cb, y_fp32 != 0, partial ? ex.splits : 1,
-                                          partial, static_cast<int*>(workspace), st),
+    r = hip_status(hx::launch_linear_mfma(ah, rs, tr, svh, y, M, K, N, bits, cb, y_fp32 != 0, ex.splits, partial,
+                                          static_cast<int*>(workspace), st),
                    "hx_exl3_gemm(mfma)");
     return r ? r : HX_GEMM_PATH_MFMA;
 }

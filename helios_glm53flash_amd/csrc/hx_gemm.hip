@@ -62,25 +62,25 @@ hipError_t launch_input_had(const _Float16* x, const _Float16* suh, _Float16* a,
     return hipGetLastError();
 }
 
-// K splits: tiles that leave more than half of the 768 resident workgroups (3 on each of 256 CUs) empty are split,
-// with at least 8 chunks of 64 k each.  A split costs its accumulators a trip through memory (written, then
-// read by the last to arrive), so past 5 splits only up to 2 workgroups per CU.  4096 -> 12288 4-bit (96 row x
-// column tiles) at M = 45 / 128: 58 / 67 us unsplit, 35.0 / 49.4 with 2, 28.8 / 42.6 with 4, 27.3 / 41.1 with 5,
-// 28.9 / 49.4 with 8; 24576 columns (192 tiles) at M = 45: 44.6 with 2, 36.5 with 4; 8192 -> 8192 (64 tiles): 63.0
-// with 2, 42.3 with 5, 37.1 with 8 (graphs of 10 calls, input transform included).
-// Where tiles alone reach more than half of the CUs a split saves less of a chunk's time, so it has to be longer to
-// be worth its trip: 16 chunks (12 at up to 32 rows, whose accumulators are few), and 24 with more tiles than CUs.
-// 4-bit, 126 rows, 17792 columns (139 tiles), unsplit / 2 splits: K = 1024 25.4 / 30.6 us, K = 1280 29.1 / 32.9,
-// K = 1536 32.8 / 35.6, K = 2048 40.8 / 40.4; 200 rows (278 tiles): K = 1024 28.9 / 36.5, K = 2048 49.5 / 48.4, K = 3072
-// 69.0 / 60.1.  (512 to 24576 columns, K = 512 to 8192, 17 to 512 rows, 2, 4 and 6 bits: no shape more than 2 %
-// slower than unsplit; with 8 chunks everywhere up to 30 %.)
+// K splits: row x column tiles that leave more than half of the 768 resident workgroups (3 on each of 256 CUs) empty,
+// split where that is faster than the unsplit tile, which sums its input itself (2, 4, 5, 6 and 8 bits, 512 to 40960
+// columns, K = 512 to 8192, 17 to 2000 rows: 4378 shapes, against the unsplit call 0.825 in the geometric mean, 2 %
+// slower or more at 9 of them; the best split of each shape would give 0.819).
+// A split costs row sums ahead of it, and its accumulators a trip through memory (written, then read by the last to
+// arrive).  The more CUs the tiles fill by themselves, the less a split saves, so K has to be the longer: in chunks
+// of 64, tiles / 4 up to 128 tiles (half of the CUs; never under 20), tiles / 3 beyond.  4-bit, M = 100: 64
+// tiles (8192 columns) K = 1024 22.0 us unsplit, 22.3 with 2 splits, K = 1280 24.9 / 22.4 with 3, K = 2048 33.0 / 26.6 with 4;
+// 139 tiles (17792 columns) K = 2048 33.8 / 36.1 with 3, K = 2560 39.5 / 39.2, K = 3072 45.0 / 41.4 with 5.
+// One workgroup per CU where 4 splits or more reach that, two if K is 6144 or longer; else at most 5.  48 tiles,
+// 8-bit, K = 3072, M = 100: 45.8 us unsplit, 30.4 with 5, 36.6 with 8.
 static int mfma_splits(int M, int K, int N)
 {
     const long tiles = (long)((M + MF_BM - 1) / MF_BM) * (N / 128), nk = K / MF_BK;
     auto least = [](long a, long b) { return a < b ? a : b; };
-    const long two = 2 * GEMV_CUS / tiles;
-    const long chunks = tiles <= GEMV_CUS / 2 ? 8 : tiles > GEMV_CUS ? 24 : M <= 32 ? 12 : 16;
-    const long s = least(least(3 * GEMV_CUS / tiles, two > 5 ? two : 5), least(nk / chunks, 8));
+    const long from = tiles <= GEMV_CUS / 2 ? (tiles + 3) / 4 : (tiles + 2) / 3;
+    if (nk < (from > 20 ? from : 20)) return 1;
+    const long round = (nk >= 96 ? 2 : 1) * GEMV_CUS / tiles;
+    const long s = least(least(3 * GEMV_CUS / tiles, round >= 4 ? round : 5), least(nk / (tiles <= 64 ? 6 : 8), 8));
     return s > 1 ? (int)s : 1;
 }
 
@@ -89,20 +89,24 @@ static size_t al256(size_t v) { return (v + 255) & ~(size_t)255; }
 // 16-column fragments of accumulators that a split of the tallest row tile stores.
 static int mfma_frags(int M) { return ((M < MF_BM ? M : MF_BM) + 15) / 16 * 2; }
 
-// A function of the shape alone, so that a shape takes the same path (and rounds alike) wherever MFMA_EXTRA_BYTES are
-// there: what does not fit those is left out even if the caller has more.
-MfmaExtra mfma_extra(int M, int K, int N)
+// Unsplit calls with row sums made ahead of the tiles (whose input then goes to LDS by buffer loads): codebook 2 at up
+// to 4 bits over 384 tiles (half of the resident workgroups) and more, where a tile's sums cost more than their
+// launch: sustained, sums ahead / in the tile, 4-bit 4096 -> 24576, M = 2000 470 / 482 us, 4096 -> 12288, M = 400 (384
+// tiles) 73.0 / 76.2, 2-bit 2048 -> 24576, M = 2000 249 / 255; but 5-bit 4096 -> 151552, M = 512 764 / 755, 5-bit 4096 ->
+// 24576, M = 2000 513 / 500, 8-bit 8192 -> 40960, M = 1500 1343 / 1283 (their trellis words take two loads a chunk), and
+// with fewer tiles 2 to 30 % longer (8-bit, 2048 -> 24576, M = 65 39.3 / 30.4).
+// A function of shape, width and codebook alone, so that a call takes the same path (and rounds alike) wherever
+// MFMA_EXTRA_BYTES are there: what does not fit those is left out even if the caller has more.
+MfmaExtra mfma_extra(int M, int K, int N, int bits, int cb)
 {
-    MfmaExtra e{al256((size_t)M * (K / 128) * sizeof(float)), 0, 1};
-    if (e.rs > MFMA_EXTRA_BYTES) return MfmaExtra{0, 0, 1};
-    const size_t one = (size_t)((M + MF_BM - 1) / MF_BM) * (N / 128) * mfma_frags(M) * MF_THREADS * sizeof(hx_f4);
+    const size_t rs = al256((size_t)M * (K / 128) * sizeof(float));
+    const long tiles = (long)((M + MF_BM - 1) / MF_BM) * (N / 128);
+    const size_t one = (size_t)tiles * mfma_frags(M) * MF_THREADS * sizeof(hx_f4);
     int s = mfma_splits(M, K, N);
-    while (s > 1 && e.rs + s * one > MFMA_EXTRA_BYTES) --s;
-    if (s > 1) {
-        e.partial = s * one;
-        e.splits = s;
-    }
-    return e;
+    while (s > 1 && rs + s * one > MFMA_EXTRA_BYTES) --s;
+    if (s > 1) return MfmaExtra{rs, s * one, s};
+    const bool ahead = cb == 2 && bits <= 4 && tiles >= 384 && rs <= MFMA_EXTRA_BYTES;
+    return MfmaExtra{ahead ? rs : 0, 0, 1};
 }
 
 hipError_t launch_linear_mfma(const _Float16* a_had, const float* rs, const uint16_t* trellis, const _Float16* svh,

@@ -109,7 +109,8 @@ __device__ __forceinline__ void linear_tile_store(const hx_f4 (&acc)[BM / 16][2]
 
 // One (row tile, column group, K split).  A split stores its raw accumulators (device-coherent 16-byte
 // stores, each lane its own), and the last split of the tile to arrive adds them in split order
-// (deterministic) in the same lanes.
+// (deterministic) in the same lanes.  EXT: the row sums of a are given, and a goes to LDS by buffer loads; else (never
+// split) codebook 2 sums its rows from a on its way through registers.
 template <int BITS, int CB, int BM, bool EXT>
 __device__ __forceinline__ void linear_tile(const MfmaGemmArgs& g, int mt, int cg, int s, MfmaSmemQ& sm)
 {
@@ -172,7 +173,7 @@ __device__ __forceinline__ void linear_tile(const MfmaGemmArgs& g, int mt, int c
 }
 
 // Quarter-operand tiles of 128 rows, the last row tile 32, 64 or 96 rows tall if that holds its rows;
-// three workgroups per CU.  EXT: the row sums of a are given, and a goes to LDS by buffer loads.
+// three workgroups per CU.
 template <int BITS, int CB, bool EXT>
 __global__ __launch_bounds__(MF_THREADS, qt_occ<CB>()) void linear_mfma_kernel(MfmaGemmArgs g)
 {
@@ -183,11 +184,9 @@ __global__ __launch_bounds__(MF_THREADS, qt_occ<CB>()) void linear_mfma_kernel(M
     if (!xcd_group_index(blockIdx.x + blockIdx.y * gridDim.x, gridDim.y, gridDim.x, mt, cs)) return;
     const int groups = g.N >> 7, cg = cs % groups, s = cs / groups;
     const int rows = g.M - mt * MF_BM;
-    if constexpr (EXT) {
-        if (rows <= 32) return linear_tile<BITS, CB, 32, EXT>(g, mt, cg, s, sm);
-        if (rows <= 64) return linear_tile<BITS, CB, 64, EXT>(g, mt, cg, s, sm);
-        if (rows <= 96) return linear_tile<BITS, CB, 96, EXT>(g, mt, cg, s, sm);
-    }
+    if (rows <= 32) return linear_tile<BITS, CB, 32, EXT>(g, mt, cg, s, sm);
+    if (rows <= 64) return linear_tile<BITS, CB, 64, EXT>(g, mt, cg, s, sm);
+    if (rows <= 96) return linear_tile<BITS, CB, 96, EXT>(g, mt, cg, s, sm);
     linear_tile<BITS, CB, MF_BM, EXT>(g, mt, cg, s, sm);
 }
 

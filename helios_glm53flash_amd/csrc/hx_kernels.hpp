@@ -31,19 +31,19 @@ hipError_t launch_linear_gemv(const _Float16* x, const uint16_t* trellis, const 
 // rs: optional [rows][K / 128] fp32 sums of the transformed blocks (MfmaExtra::rs).
 hipError_t launch_input_had(const _Float16* x, const _Float16* suh, _Float16* a, float* rs, long rows, int K,
                             hipStream_t st);
-// rs (null: slower tiles that sum the input themselves) and, with splits > 1, partial and counter are
-// workspace (MfmaExtra; the arrival counters are zero before the call and left at zero).
+// rs (null: the tiles sum the input themselves) and, with splits > 1, partial and counter are workspace (MfmaExtra;
+// the arrival counters are zero before the call and left at zero).
 hipError_t launch_linear_mfma(const _Float16* a_had, const float* rs, const uint16_t* trellis, const _Float16* svh,
                               void* y, int M, int K, int N, int bits, int cb, bool y_fp32, int splits, void* partial,
                               int* counter, hipStream_t st);
-// What makes the MFMA path fastest beyond the memory that it needs: row sums of the input, then K-split partials.  At
-// most 768 workgroups of 128 x 128 fp32 partials (48 MiB, when few tiles are split) and K M / 32 bytes of row sums.
+// What a call uses beyond the memory that it needs: row sums of the input, then K-split partials.  At most 768
+// workgroups of 128 x 128 fp32 partials (48 MiB, when few tiles are split) and K M / 32 bytes of row sums.
 constexpr size_t MFMA_EXTRA_BYTES = 64u << 20;
 struct MfmaExtra {
     size_t rs, partial;  // bytes (0: done without)
     int splits;
 };
-MfmaExtra mfma_extra(int M, int K, int N);
+MfmaExtra mfma_extra(int M, int K, int N, int bits, int cb);
 
 // utilities (hx_misc.hip)
 hipError_t launch_reconstruct(_Float16* out, const uint16_t* packed, int packed_rows, int packed_cols,

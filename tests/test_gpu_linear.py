@@ -159,7 +159,7 @@ def test_mfma_small_workspace(hx, ws_bytes):
 
 @pytest.mark.parametrize("M,N", [(45, 512), (300, 256)])
 def test_mfma_workspace_beyond_the_least(hx, M, N):
-    """Without a_had: the least workspace, room for the row sums, one byte short of the K-split partials, and enough
+    """Without a_had: the least workspace, room for the row sums of K splits, one byte short of their partials, and enough
     for them.  Nothing past the end is written, the counters return to zero."""
     import ctypes as C
     import torch
@@ -173,8 +173,8 @@ def test_mfma_workspace_beyond_the_least(hx, M, N):
     xd, gw = _dev(x), w.c()
     least = lib.hx_exl3_gemm_workspace_size(M, N, K)
     rs = (M * K // 32 + 255) // 256 * 256  # an fp32 sum per 128 inputs
-    # 2048 / 64 = 32 chunks of k: 4 splits of 8; a split stores 16-row fragments of 128 columns, a row tile at most 128 rows
-    partial = (M + 127) // 128 * (N // 128) * 4 * ((min(M, 128) + 15) // 16 * 16) * 128 * 4
+    # 2048 / 64 = 32 chunks of k: 5 splits of 6 and 7; a split stores 16-row fragments of 128 columns, a row tile at most 128 rows
+    partial = (M + 127) // 128 * (N // 128) * 5 * ((min(M, 128) + 15) // 16 * 16) * 128 * 4
     outs = []
     for n in (least, least + rs, least + rs + partial - 1, least + rs + partial,
               least + lib.hx_exl3_gemm_extra_bytes()):
@@ -187,18 +187,19 @@ def test_mfma_workspace_beyond_the_least(hx, M, N):
         assert_close(y.cpu().numpy(), ref, what=f"workspace of {n}")
         assert bool((ws[n:] == 7).all()) and not bool(ws[:64 * 1024].any())
         outs.append(y)
-    assert torch.equal(outs[1], outs[2]) and torch.equal(outs[3], outs[4]) and not torch.equal(outs[2], outs[3])
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[1], outs[2]) and torch.equal(outs[3], outs[4])
+    assert not torch.equal(outs[2], outs[3])
     ws = torch.zeros(least, dtype=torch.uint8, device="cuda")
     assert lib.hx_exl3_gemm(outs[0].data_ptr(), xd.data_ptr(), C.byref(gw), M, N, K, bits, 1, None, None, 0,
                             ws.data_ptr(), 64 * 1024) == HX_ERR_WORKSPACE
 
 
 @pytest.mark.parametrize("M,K,N,split", [(126, 1280, 17792, False), (512, 1024, 8192, False), (200, 2048, 17792, False),
-                                         (17, 1280, 24576, False), (126, 1280, 8192, True), (17, 1536, 17792, True),
-                                         (126, 2048, 17792, True), (384, 3072, 12288, True)])
+                                         (17, 1280, 24576, False), (126, 2944, 17792, False), (126, 1280, 8192, True),
+                                         (17, 3072, 17792, True), (45, 4096, 12288, True), (200, 6144, 12288, True)])
 def test_mfma_splits_only_where_they_pay(hx, M, K, N, split):
-    """Tiles on more than half of the CUs are split only if a split is long enough (shorter ones were up to 30 % slower
-    than no split): with room for the row sums alone the call is unsplit, with more room it is split or the same."""
+    """Splits of a K that is too short for its number of tiles were up to 30 % slower than no split: with the least
+    workspace the call is unsplit, with more room it is split, or, where K is too short, gives the same bits."""
     import ctypes as C
     import torch
     from helios_glm53flash_amd._lib import lib
@@ -207,7 +208,7 @@ def test_mfma_splits_only_where_they_pay(hx, M, K, N, split):
     xd, gw = _dev(make_x(52, M, K)), w.c()
     least = lib.hx_exl3_gemm_workspace_size(M, N, K)
     ys = []
-    for n in (least + (M * K // 32 + 255) // 256 * 256, least + lib.hx_exl3_gemm_extra_bytes()):
+    for n in (least, least + lib.hx_exl3_gemm_extra_bytes()):
         ws = torch.zeros(n, dtype=torch.uint8, device="cuda")
         y = torch.empty((M, N), device="cuda")
         lib.hx_exl3_gemm(y.data_ptr(), xd.data_ptr(), C.byref(gw), M, N, K, 2, 1, None, None, 0, ws.data_ptr(), n)
@@ -215,6 +216,32 @@ def test_mfma_splits_only_where_they_pay(hx, M, K, N, split):
         ys.append(y)
     assert torch.equal(*ys) == (not split)
     assert float((ys[0] - ys[1]).norm() / ys[0].norm()) < 1e-5  # the order of fp32 sums: sqrt(K) * 2^-24 = 4e-6 of the size
+
+
+@pytest.mark.parametrize("M,bits", [(130, 4), (170, 3), (200, 2), (256, 1), (256, 5)])
+def test_mfma_many_tiles(hx, M, bits):
+    """384 tiles: up to 4 bits with the row sums made ahead of the tiles if the workspace has room for them, in the tile
+    otherwise; last row tiles of every height."""
+    import ctypes as C
+    import torch
+    from oracle import oracle as O
+    from helios_glm53flash_amd._lib import lib
+    K, N = 128, 24576
+    tr, suh, svh = make_linear(61, K, N, bits)
+    x = make_x(62, M, K)
+    w = hx.GroupWords(_dev(tr, torch.int16), _dev(suh), _dev(svh), hx.MUL1)
+    ref = O.linear(x, tr, suh, svh, K, N, bits, 2, out_f16=False)
+    xd, gw = _dev(x), w.c()
+    least = lib.hx_exl3_gemm_workspace_size(M, N, K)
+    for room in (0, (M * K // 32 + 255) // 256 * 256):
+        ws = torch.zeros(least + room + 4096, dtype=torch.uint8, device="cuda")
+        y = torch.empty((M, N), device="cuda")
+        lib.hx_exl3_gemm(y.data_ptr(), xd.data_ptr(), C.byref(gw), M, N, K, bits, 1, None, None, 0, ws.data_ptr(),
+                         least + room)
+        torch.cuda.synchronize()
+        assert_close(y.cpu().numpy(), ref, what=f"room {room}")
+        sums = ws[least:least + room].view(torch.float32)
+        assert bool(sums.any()) == (room > 0 and bits <= 4) and not bool(ws[least + room:].any())
 
 
 def test_mfma_captured_on_a_decode_stream(hx):
