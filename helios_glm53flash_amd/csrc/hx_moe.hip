@@ -180,8 +180,8 @@ size_t decode_lds_pad(const void* kernel, size_t lds, int max_per_cu)
 // 2 per group, 72.6 with 1; 3 tokens 83.7 with 1 (85.5 with 1024 units over its 800 groups); 4 tokens 102 with
 // 1 (2, 3 and 4 were slower already); 8 tokens 214 with 2, 243 with 4.  64 experts, 2048 x 1024, 2 tokens: 34.0
 // with 2, 37.7 with 3, 45.5 with 4.
-// A phase of few column groups gets more than 2, up to 512 units (768 from 5 tokens on) of at least 4 (8) k blocks:
-// with 2 it leaves CUs empty.  At most 2 / 3 / 4 / 8 per group: 4096 x 256, 288 experts, top-8: 2 tokens (68 gate/up
+// A phase of few column groups gets more than 2, up to 512 units (768 from 5 tokens on) of at least 4 (8) k blocks, and up
+// to 256 units of 2 blocks: with 2 per group it leaves CUs empty.  At most 2 / 3 / 4 / 8 per group: 4096 x 256, 288 experts, top-8: 2 tokens (68 gate/up
 // groups) 42.3 / 39.7 / 38.4 / 38.2 us, 4 tokens (132) 50.9 / 43.9 / 45.8 / 50.9, 5 tokens (164) 63.0 / 61.5 / 59.7 / 62.9,
 // 6 tokens (196) 69.3 / 64.9 / 63.7 / 66.3; 7168 x 256, 128 experts: 3 tokens (100) 60.9 / 55.5 / 53.2 / 51.7; 2048 x
 // 768, 64 experts, top-4: 2 tokens (108) 28.6 / 27.5 / 27.5 / 35.3, 4 tokens (204) 33.1 / 33.7 / 38.1 / 40.5, 6 tokens
@@ -198,9 +198,10 @@ int decode_units(MoeDecodeArgs& a, int resident)
         const long mt = a.T <= 4 ? 4 : 8;
         auto per_group = [&](long cg, long kb) {
             auto least = [](long p, long q) { return p < q ? p : q; };
+            auto most = [](long p, long q) { return p > q ? p : q; };
             const long fit = (kb * 128 * mt * 2 + 32767) / 32768, near = (2 * resident + cg) / (2 * cg);
-            const long few = least((mt == 4 ? 512 : 768) / cg, kb / mt), round = least(near, few > 2 ? few : 2);
-            return fit > round ? fit : round;
+            const long few = most(least((mt == 4 ? 512 : 768) / cg, kb / mt), least(256 / cg, kb / 2));
+            return most(fit, least(near, most(few, 2)));
         };
         ug = cg_gu * per_group(cg_gu, kb_gu);
         ud = cg_d * per_group(cg_d, kb_d);
