@@ -37,6 +37,7 @@ struct Prof {
     }
 };
 Prof g_prof;
+// "shared_expert" keeps its index and reads 0: its GEMMs are jobs of the gate/up and down phases.
 const char* const k_phase_names[] = {"route", "permute", "experts_gate_up", "experts_down", "combine",
                                      "shared_expert", "prefill_plan_gather", "prefill_gemm_gate_up",
                                      "prefill_guad", "prefill_gemm_down", "prefill_combine", "moe_decode"};
@@ -666,20 +667,14 @@ int hx_moe_layer(void* y, float* y_routed, const void* x, const void* scores, co
             a.out_w = wt;
         } else {
             // Routed and sorted once ahead of the layer kernel: its 2000-4000 workgroups would each select for 5-8
-            // tokens and rank up to 64 routes (8 tokens 272 -> 214 us; at 2-4 tokens the two launches cost more
-            // than they save, 102 -> 111 us).
+            // tokens and rank up to 64 routes (8 tokens 272 -> 211 us, 288 experts, 4096 x 2048; at 2-4 tokens routing
+            // ahead in two launches took longer, 4 tokens 102 -> 111).
             {
                 Phase ph(0, st);
-                r = hip_status(hx::launch_routing(static_cast<const _Float16*>(scores),
-                                                  static_cast<const _Float16*>(bias), idx, wt, tokens, num_experts,
-                                                  topk, routed_scale, st),
+                r = hip_status(hx::launch_route_few(static_cast<const _Float16*>(scores),
+                                                    static_cast<const _Float16*>(bias), tokens, num_experts, topk,
+                                                    routed_scale, idx, wt, cnt, ts, wsorted, r2s, st),
                                "hx_moe_layer(routing)");
-            }
-            if (r) return r;
-            {
-                Phase ph(1, st);
-                r = hip_status(hx::launch_permute(idx, wt, tokens, topk, num_experts, cnt, ts, wsorted, r2s, nullptr, st),
-                               "hx_moe_layer(permute)");
             }
             if (r) return r;
             a.expert_count = cnt;

@@ -64,7 +64,7 @@ hipError_t launch_input_had(const _Float16* x, const _Float16* suh, _Float16* a,
 
 // K splits: row x column tiles that leave more than half of the 768 resident workgroups (3 on each of 256 CUs) empty,
 // split where that is faster than the unsplit tile, which sums its input itself (2, 4, 5, 6 and 8 bits, 512 to 40960
-// columns, K = 512 to 8192, 17 to 2000 rows: 4378 shapes, against the unsplit call 0.825 in the geometric mean, 2 %
+// columns, K = 512 to 8192, 17 to 2000 rows: 4378 shapes, against the unsplit call 0.823 in the geometric mean, 2 %
 // slower or more at 9 of them; the best split of each shape would give 0.819).
 // A split costs row sums ahead of it, and its accumulators a trip through memory (written, then read by the last to
 // arrive).  The more CUs the tiles fill by themselves, the less a split saves, so K has to be the longer: in chunks

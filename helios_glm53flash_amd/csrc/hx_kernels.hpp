@@ -58,6 +58,11 @@ hipError_t launch_routing(const _Float16* scores, const _Float16* bias, int64_t*
 hipError_t launch_permute(const int64_t* ids, const _Float16* w, int M, int topk, int E, int64_t* expert_count,
                           int64_t* token_sorted, _Float16* weight_sorted, int64_t* route_to_sorted,
                           int64_t* workspace, hipStream_t st);
+// launch_routing (with top-k on the biased key) and launch_permute for up to 8 tokens and 64 routes in one launch
+// (hx_moe.hip).
+hipError_t launch_route_few(const _Float16* scores, const _Float16* bias, int T, int E, int topk, float scale, int64_t* idx,
+                            _Float16* w, int64_t* expert_count, int64_t* token_sorted, _Float16* weight_sorted,
+                            int64_t* route_to_sorted, hipStream_t st);
 // Chunked permutation for many routes (same result as launch_permute): scratch holds
 // 2 * ceil(M*topk/1024) * E ints, arrive is a zero-initialised counter (left zero).
 hipError_t launch_permute_chunked(const int64_t* ids, const _Float16* w, int M, int topk, int E, int64_t* expert_count,

@@ -1,7 +1,7 @@
 // hx_moe_decode.hpp -- fused MoE layer for few tokens (T <= 8, T*topk <= 64) on gfx950 in ONE
 // launch, without host synchronisation.  Every workgroup computes the router top-k and the
-// token-by-expert permutation from the fp16 scores (a few hundred bytes; the layer calls it with the
-// caller's or an already built permutation from 5 tokens on), then runs one unit:
+// token-by-expert permutation from the fp16 scores (a few hundred bytes; from 5 tokens on it reads the
+// caller's permutation, or the one that the layer builds ahead of it), then runs one unit:
 //
 //   gate/up unit  one k range of one expert's gate or up GEMV with the trellis decode fused; the
 //                 last-arriving unit of a (slot, column group) adds the partial sums, runs the
@@ -34,7 +34,7 @@ constexpr int DEC_STATUS_BAD_BITS = 2; // a per-expert bit table held a width ou
 // svh of up, suh of down; down units: svh of down).
 constexpr int DEC_TABS = 5;
 // Expert table entries parked in LDS while the plan is built (for up to this many experts): they use the input
-// rows' dynamic LDS, which is written only after the barrier that follows the plan.  An array of their own
+// rows' dynamic LDS, which is written only behind a further barrier of the unit (see build_plan's end).  An array of their own
 // (12.8 KB) held the 4-row kernel at 3 workgroups per CU instead of 4 and the 8-row kernel at 2: the layer at
 // 4 tokens 110 -> 102 us, at 8 tokens 464 -> 272 us.
 constexpr int DEC_TAB_MAX_E = 320;
@@ -241,6 +241,21 @@ HX_INLINE void wave_topk(const _Float16* scores, const _Float16* bias, int E, in
     w_out = (float)(_Float16)(w_out * scale / sum);
 }
 
+// Rank of this lane's route (expert ei; lanes past R hold no route) among the R <= 64 routes of a wave, for a stable
+// counting sort by expert: routes of lower experts, routes of the same expert on lower lanes, routes of the
+// same expert.  Route j is read from lane j; lanes 0..R-1 have to be active.
+HX_INLINE void rank_route(int ei, int R, int& less, int& eqb, int& cnt)
+{
+    const int i = threadIdx.x & 63;
+    less = eqb = cnt = 0;
+    for (int j = 0; j < R; ++j) {
+        const int ej = __builtin_amdgcn_readlane(ei, j);
+        less += ej < ei;
+        eqb += (ej == ei) && (j < i);
+        cnt += ej == ei;
+    }
+}
+
 // Element `i` of a 3-array member of the kernel arguments, by selects rather than a run-time index:
 // indexing an argument array at run time makes the compiler copy the whole argument block into
 // per-lane scratch memory.
@@ -316,7 +331,7 @@ HX_INLINE void load_slot_tables(const MoeDecodeArgs& a, SlotTables& t, int e, in
 
 // Build the plan in LDS (every workgroup computes the same plan), and the tables of projection
 // proj of the workgroup's own slot: routed slot my_slot >= 0 if it is active, the shared expert for
-// my_slot == DEC_SHARED, none for -1.  Layer mode routes the tokens; grouped mode reads the caller's
+// my_slot == DEC_SHARED, none for -1.  With a.scores (up to 4 tokens) it routes the tokens; without, it reads
 // expert_count / token_sorted / weight_sorted.
 template <int MT>
 __device__ __forceinline__ void build_plan(const MoeDecodeArgs& a, DecodePlan& p, int my_slot, int proj,
@@ -328,7 +343,8 @@ __device__ __forceinline__ void build_plan(const MoeDecodeArgs& a, DecodePlan& p
     uint64_t (*tab_lds)[TAB_MAX_E] = reinterpret_cast<uint64_t (*)[TAB_MAX_E]>(a_lds);  // table entries of every expert
     const int wave = hx_vwave(), lane = threadIdx.x & 63;
     const int R = a.T * a.topk;
-    if (a.scores) {
+    const bool route = MT <= 4 && a.scores != nullptr;
+    if (route) {
         // The slot's table entries would be one more dependent load after the ranking.  Instead
         // they are loaded for every expert while the scores are in flight and parked in LDS: wave 0
         // loads trellis and suh (parked after its selection, which then waits for the scores only,
@@ -418,12 +434,7 @@ __device__ __forceinline__ void build_plan(const MoeDecodeArgs& a, DecodePlan& p
                 cnt = 1;
                 n = R;
             } else {
-                for (int j = 0; j < R; ++j) {
-                    const int ej = __builtin_amdgcn_readlane(ei, j);
-                    less += ej < ei;
-                    eqb += (ej == ei) && (j < i);
-                    cnt += ej == ei;
-                }
+                rank_route(ei, R, less, eqb, cnt);
                 const uint64_t fm = __ballot(i < R && eqb == 0);  // first selection of each expert
                 for (int j = 0; j < R; ++j)                        // distinct experts below ei
                     if ((fm >> j) & 1) dless += __builtin_amdgcn_readlane(ei, j) < ei;
@@ -498,8 +509,10 @@ __device__ __forceinline__ void build_plan(const MoeDecodeArgs& a, DecodePlan& p
         }
     }
     __syncthreads();
-    // the slot's epilogue tables (the epilogues read them after later barriers)
-    if (a.scores && hx_vtid() == 0 && my_slot >= 0 && my_slot < p.n && a.E <= TAB_MAX_E) {
+    // the slot's epilogue tables (the epilogues read them after later barriers).  They are read from the input rows' LDS:
+    // the barrier ahead of the first input_store or input_copy (gu_segment's, d_segment's wait_inputs) keeps those
+    // writes behind this read.
+    if (route && hx_vtid() == 0 && my_slot >= 0 && my_slot < p.n && a.E <= TAB_MAX_E) {
         const int e = p.expert[my_slot];
 #pragma unroll
         for (int q = 2; q < DEC_TABS; ++q) {

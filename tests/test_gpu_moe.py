@@ -421,3 +421,29 @@ def test_decode_few_column_groups(hx, T, topk, E, hidden, inter):
     """Phases of few column groups: 3 to 8 units per group, k ranges of unequal length among them."""
     for _ in range(2):
         _run_layer(hx, E, hidden, inter, topk, T, 2, 2, seed=T + hidden)
+
+
+@pytest.mark.parametrize("T,topk,E,bias", [(5, 1, 1, False), (5, 12, 12, True), (6, 10, 100, False), (8, 8, 512, True),
+                                           (7, 9, 511, False), (8, 8, 8, True)])
+def test_route_few_tokens(hx, T, topk, E, bias):
+    """Routing and permutation of 5 to 8 tokens in one launch, with equal scores (ties go to the lower expert), both
+    infinities and fp16's lowest value among them."""
+    import torch
+    from oracle import oracle as O
+    exl3, moe = hx
+    hidden, inter = 128, 128
+    ex = moe.ExpertSet.synthetic(E, hidden, inter, 2, seed=T + E)
+    layer = moe.MoeLayer(ex, None, topk=topk)
+    r = np.random.default_rng(T * E)
+    x = r.standard_normal((T, hidden)).astype(np.float16)
+    scores = (np.round(r.standard_normal((T, E)) * 4) / 4).astype(np.float16)
+    if E > 4:
+        scores[0, :4] = np.inf, -np.inf, -65504, 65504
+    b = (np.round(r.standard_normal(E)) / 8).astype(np.float16) if bias else None
+    y_routed = torch.empty((T, hidden), dtype=torch.float32, device="cuda")
+    layer(torch.from_numpy(x).cuda(), torch.from_numpy(scores).cuda(), y_routed=y_routed,
+          bias=torch.from_numpy(b).cuda() if bias else None)
+    torch.cuda.synchronize()
+    idx, w = O.routing(scores, topk, 2.5, b)
+    ref, _ = O.moe_rows(x, hidden, inter, idx, w, np.arange(T), _oracle_experts(ex, set(range(E))), None, 10.0)
+    assert_close(y_routed.cpu().numpy(), ref, what=f"T={T} E={E}")
