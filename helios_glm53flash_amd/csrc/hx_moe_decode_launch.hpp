@@ -15,14 +15,30 @@ static hipError_t launch_k(Kernel kernel, const MoeDecodeArgs& a0, hipStream_t s
 {
     MoeDecodeArgs a = a0;
     const void* k = reinterpret_cast<const void*>(kernel);
-    size_t lds = (size_t)MT * 1024 * sizeof(_Float16);
-    for (int it = 0; it < 4; ++it) {
-        const size_t need = (size_t)MT * decode_units(a, decode_resident(k, DEC_THREADS, lds, 4)) * sizeof(_Float16);
-        if (need == lds) break;
-        lds = need;
+    // The plan of this thread's last launch serves the next one of the same kernel and shape on the same device (the
+    // layers of a decode step).  Host time of a one-token layer call from C++: mean 8.5, at most 10.2 us in 14 runs without,
+    // 8.2 and 9.2 in 10 runs with it (5.5 to 9 us by the run).
+    struct Plan {
+        const void* kernel;
+        int dev, T, hidden, inter, slots, units_gu, units_d;
+        size_t lds;
+    };
+    static thread_local Plan p{};
+    int dev = 0;
+    if (hipError_t e = hipGetDevice(&dev)) return e;
+    if (p.kernel != k || p.dev != dev || p.T != a.T || p.hidden != a.hidden || p.inter != a.inter || p.slots != a.routed_slots) {
+        size_t lds = (size_t)MT * 1024 * sizeof(_Float16);
+        for (int it = 0; it < 4; ++it) {
+            const size_t need = (size_t)MT * decode_units(a, decode_resident(k, DEC_THREADS, lds, 4)) * sizeof(_Float16);
+            if (need == lds) break;
+            lds = need;
+        }
+        lds = decode_lds_pad(k, lds > DEC_TAB_LDS ? lds : DEC_TAB_LDS, 4);
+        p = Plan{k, dev, a.T, a.hidden, a.inter, a.routed_slots, a.units_gu, a.units_d, lds};
     }
-    lds = decode_lds_pad(k, lds > DEC_TAB_LDS ? lds : DEC_TAB_LDS, 4);
-    hipLaunchKernelGGL(kernel, dim3(a.units_gu + a.units_d), dim3(DEC_THREADS), lds, st, a);
+    a.units_gu = p.units_gu;
+    a.units_d = p.units_d;
+    hipLaunchKernelGGL(kernel, dim3(a.units_gu + a.units_d), dim3(DEC_THREADS), p.lds, st, a);
     return hipGetLastError();
 }
 
