@@ -1,7 +1,7 @@
 // hx_mfma.hpp -- EXL3 decode + MFMA tile core for gfx950 (M > 16 paths: the dense linear and the
 // grouped expert GEMMs of the prefill), and the Hadamard-128 transform on the matrix cores.
 //
-// Workgroup = 4 waves, output tile BM x 128 (BM = 128, 64 or 32; 128 columns = one Hadamard block),
+// Workgroup = 4 waves, output tile BM x 128 (BM = 128, 96, 64 or 32; 128 columns = one Hadamard block),
 // K consumed in chunks of 64.  Each wave owns 32 output columns for all BM rows and decodes those
 // columns' trellis words itself, straight into MFMA B operands (mfma_tile_q below); only A (the
 // input-transformed activations) goes through LDS, one barrier per chunk: qt_pf(BM) chunks ahead, by

@@ -77,9 +77,10 @@ __global__ __launch_bounds__(256) void gemv_nt_kernel(const _Float16* x, const _
 // wave per 32 x 32 block over all of K waited a round trip of latency every few steps (115 us at
 // 4096 x 288 x 4096, 27 us at M = 16).  A wave has NB chunks of 64 k in LDS buffers of its own, filled
 // by buffer loads with an LDS destination (8 rows x 128 bytes each): no barrier, only its own loads to
-// wait for.  What bounds it is a CU's read path from L2: whole 128-byte lines come at 115 GB/s
-// per CU, the 64-byte halves that fragments loaded straight into MFMA layout touch at 37 GB/s (that
-// variant of this kernel: 45 us at M = 4096, 17 us at M = 33-512).
+// wait for.  What bounds it is these loads: 24.9 us at 4096 x 288 x 4096, 22.0 without the MFMAs, 24.1 without the
+// LDS reads, 21.7 with neither (251 MB through 192 CUs, 60 GB/s each; at M = 512 8.4 / 7.9 / 8.0 / 7.7, and nothing at
+// 64 experts).  In whole 128-byte lines a CU reads up to 115 GB/s from L2, in the 64-byte halves that fragments loaded
+// straight into MFMA layout touch 37 GB/s (that variant of this kernel: 45 us at M = 4096, 17 us at M = 33-512).
 // LDS rows are 64 halves with the 16-byte chunks of row r permuted by mf_swz(r) (hx_mfma.hpp).
 // DMA false: x or w is not 16-byte aligned, which the buffer loads into LDS ask for; the chunks go through
 // registers (global loads take any address), without loads in flight across chunks.
