@@ -90,11 +90,19 @@ static size_t al256(size_t v) { return (v + 255) & ~(size_t)255; }
 static int mfma_frags(int M) { return ((M < MF_BM ? M : MF_BM) + 15) / 16 * 2; }
 
 // Unsplit calls with row sums made ahead of the tiles (whose input then goes to LDS by buffer loads): codebook 2 at up
-// to 4 bits over 384 tiles (half of the resident workgroups) and more, where a tile's sums cost more than their
-// launch: sustained, sums ahead / in the tile, 4-bit 4096 -> 24576, M = 2000 470 / 482 us, 4096 -> 12288, M = 400 (384
-// tiles) 73.0 / 76.2, 2-bit 2048 -> 24576, M = 2000 249 / 255; but 5-bit 4096 -> 151552, M = 512 764 / 755, 5-bit 4096 ->
-// 24576, M = 2000 513 / 500, 8-bit 8192 -> 40960, M = 1500 1343 / 1283 (their trellis words take two loads a chunk), and
-// with fewer tiles 2 to 30 % longer (8-bit, 2048 -> 24576, M = 65 39.3 / 30.4).
+// to 4 bits.  It saves VALU work, which pays while 3 workgroups share a CU, but a chunk then takes longer for a
+// workgroup that has its CU almost to itself.  So the last round of tiles decides (768 a round), the less the more
+// full rounds there are.  Sustained, sums ahead over sums in the tile, 4-bit, K = 4096, M = 512: 384 tiles 1.09, 512 1.03,
+// 544 0.97, 768 0.98; 784 1.08, 960 1.04, 1088 1.01, 1152 1.00, 1280 0.99, 1536 0.98; 1568 1.02, 1632 1.00, 1728 0.97; 2304 and
+// more 0.97-0.99 (the same within 0.03 at 2 and 3 bits, K = 2048 and 8192, M = 256 and 1024).  More bits (two loads of
+// trellis words a chunk): 5-bit 4096 -> 151552, M = 512 1.02, 4096 -> 24576, M = 2000 1.02, 8-bit 8192 -> 40960, M = 1500 1.05.
+static bool sums_ahead(long tiles, int bits)
+{
+    constexpr long ROUND = 3 * GEMV_CUS;
+    const long full = tiles / ROUND, last = tiles % ROUND;
+    return bits <= 4 && (last == 0 || last > (full == 0 ? 512 : full == 1 ? 383 : full == 2 ? 111 : 0));
+}
+
 // A function of shape, width and codebook alone, so that a call takes the same path (and rounds alike) wherever
 // MFMA_EXTRA_BYTES are there: what does not fit those is left out even if the caller has more.
 MfmaExtra mfma_extra(int M, int K, int N, int bits, int cb)
@@ -105,7 +113,7 @@ MfmaExtra mfma_extra(int M, int K, int N, int bits, int cb)
     int s = mfma_splits(M, K, N);
     while (s > 1 && rs + s * one > MFMA_EXTRA_BYTES) --s;
     if (s > 1) return MfmaExtra{rs, s * one, s};
-    const bool ahead = cb == 2 && bits <= 4 && tiles >= 384 && rs <= MFMA_EXTRA_BYTES;
+    const bool ahead = cb == 2 && sums_ahead(tiles, bits) && rs <= MFMA_EXTRA_BYTES;
     return MfmaExtra{ahead ? rs : 0, 0, 1};
 }
 

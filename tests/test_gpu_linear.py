@@ -218,15 +218,16 @@ def test_mfma_splits_only_where_they_pay(hx, M, K, N, split):
     assert float((ys[0] - ys[1]).norm() / ys[0].norm()) < 1e-5  # the order of fp32 sums: sqrt(K) * 2^-24 = 4e-6 of the size
 
 
-@pytest.mark.parametrize("M,bits", [(130, 4), (170, 3), (200, 2), (256, 1), (256, 5)])
-def test_mfma_many_tiles(hx, M, bits):
-    """384 tiles: up to 4 bits with the row sums made ahead of the tiles if the workspace has room for them, in the tile
-    otherwise; last row tiles of every height."""
+@pytest.mark.parametrize("M,N,bits,ahead", [(130, 34816, 4, True), (170, 34816, 3, True), (200, 34816, 2, True),
+                                            (256, 34816, 1, True), (256, 34816, 5, False), (130, 24576, 4, False)])
+def test_mfma_many_tiles(hx, M, N, bits, ahead):
+    """544 tiles, up to 4 bits: the row sums made ahead of the tiles if the workspace has room for them; in the tile
+    otherwise, at more bits and at 384 tiles; last row tiles of every height."""
     import ctypes as C
     import torch
     from oracle import oracle as O
     from helios_glm53flash_amd._lib import lib
-    K, N = 128, 24576
+    K = 128
     tr, suh, svh = make_linear(61, K, N, bits)
     x = make_x(62, M, K)
     w = hx.GroupWords(_dev(tr, torch.int16), _dev(suh), _dev(svh), hx.MUL1)
@@ -241,7 +242,7 @@ def test_mfma_many_tiles(hx, M, bits):
         torch.cuda.synchronize()
         assert_close(y.cpu().numpy(), ref, what=f"room {room}")
         sums = ws[least:least + room].view(torch.float32)
-        assert bool(sums.any()) == (room > 0 and bits <= 4) and not bool(ws[least + room:].any())
+        assert bool(sums.any()) == (room > 0 and ahead) and not bool(ws[least + room:].any())
 
 
 def test_mfma_captured_on_a_decode_stream(hx):
